@@ -27,6 +27,7 @@
 #include <string.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "qmla.h"
 #include "qmla_common.h"
@@ -747,148 +748,162 @@ __global__ __launch_bounds__(256) void combine_kernel(const KParams p, int dv) {
   }
 }
 
-// LSE-weighted combine, balanced mode: one 256-thread workgroup per (query row, block of CH_HB
-// heads). Request b's partials sit in slots w + b for the workgroups w0..w1 that touched it; a
-// request covered by one workgroup was finished by the partial pass and is skipped here. Every
-// thread owns two adjacent output columns of the CH_HB heads and combines the segments CH_NS at a
-// time with a running maximum: the segment LSEs (the same for all threads) and the partial outputs
-// of a batch are loaded together, so a batch costs one memory round trip and no barrier. Two heads
-// per workgroup: at 128 x 24 rows the merge took 11.0 us against 11.9 (4 heads) and 15.1 (8 heads).
-constexpr int CH_HB = 2;
-constexpr int CH_NS = 4;   // segments per batch of loads
-// the columns of one (row, head block): H = fp16 partials without the fp8 scale, osc applies it;
-// NC adjacent columns per thread (2, or 8 for the wide latent rows, whose partials are then read
-// 16 or 32 bytes a load instead of 4 or 8, in one pass over the columns instead of four), NS
-// segments per batch of loads
-template <bool H, int NC, int HB, int NS = CH_NS>
-__device__ __forceinline__ void combine_cols(const KParams& p, int dv, int row, int jq, int req, int h0, int nh,
-                                             int w0, int nseg) {
-  const int tid = threadIdx.x;
+// LSE-weighted combine, balanced mode. Request b's partials sit in slots w + b for the workgroups
+// w0..w1 that touched it; a request covered by one workgroup was finished by the partial pass and is
+// skipped here. The merge moves few bytes; what bounds it is the number of waves launched (1536 / 3072
+// workgroups of 8 waves took 17 / 31 us for work that 4 waves each finish in 6) and the latency of its
+// dependent loads (plan, then partials). So a wave merges a chunk of 64*NC columns of one (row, head)
+// with 16 bytes a lane of fp16 partials (32 of fp32) and up to 8 segments in flight at once:
+//   SPLIT false  a wave merges its chunk alone, without LDS or a barrier (2 and 4 heads a wave, 4
+//                segments of each in flight: FP8 B 128 6.4 -> 8.4 us, GLA-g2 7.4 -> 10.0);
+//   SPLIT true   the segments of a chunk are dealt out over several waves, whose sums meet in LDS:
+//                for few rows, whose requests were split over many workgroups (one request of 1300
+//                tokens: 21 segments).
+// Combine launch before (256 threads for a row and 2 heads, 4 bytes a lane) and now: FP8 B 128 9.8 ->
+// 6.4 us, GLA-g2 11.2 -> 7.4, one request 8.6 -> 5.1, bf16 B 4 9.7 -> 4.3, 23 rank-768 requests 18.4 ->
+// 7.9, 19 rank-1792 requests 8.9 -> 8.4.
+constexpr int CM_MW = 8;    // waves of a workgroup that splits chunks, at most
+constexpr int CM_AW = 4;    // waves of a workgroup that does not
+
+// merges segments s0, s0 + step, ... (NS of them; those past nseg weigh 0 and re-read the last one)
+// into the running (m, l, a) of columns col .. col + NC of partial row rl
+template <bool H, int NC, bool VEC, int NS>
+__device__ __forceinline__ void merge_batch(const KParams& p, int64_t slot0, int64_t nrow, int rl, int dv, int col,
+                                            int s0, int step, int nseg, float& m, float& l, float (&a)[NC]) {
+  using T = std::conditional_t<H, _Float16, float>;
+  typedef __attribute__((__vector_size__(NC * sizeof(T)))) T vt;
+  float ls[NS];
+  vt v[NS];
+#pragma unroll
+  for (int k = 0; k < NS; ++k) {
+    const int s = s0 + k * step;
+    const int64_t slot = slot0 + (s < nseg ? s : nseg - 1);
+    ls[k] = s < nseg ? p.part_lse[slot * nrow + rl] : kNegInf;
+    // fp16 partials: the slot's rows at the start of its (fp32-sized) area
+    const T* src = reinterpret_cast<const T*>(p.part_o + slot * nrow * (int64_t)dv) + (int64_t)rl * dv;
+    if constexpr (VEC) {
+      v[k] = *reinterpret_cast<const vt*>(src + col);
+    } else {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) v[k][c] = src[col + c < dv ? col + c : dv - 1];
+    }
+  }
+  // segments without tokens (lse -inf) weigh 0 and a batch of them only is skipped; a NaN lse (fmaxf
+  // skips it) weighs NaN, so a row whose inputs hold a NaN merges to NaN
+  float mm = m;
+  bool live = false;
+#pragma unroll
+  for (int k = 0; k < NS; ++k) {
+    mm = fmaxf(mm, ls[k]);
+    live |= !is_neg_inf(ls[k]);
+  }
+  if (!live) return;
+  const float sc = m == kNegInf ? 0.f : __expf(m - mm);
+  l *= sc;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) a[c] *= sc;
+#pragma unroll
+  for (int k = 0; k < NS; ++k) {
+    const float wgt = is_neg_inf(ls[k]) ? 0.f : __expf(ls[k] - mm);
+    l += wgt;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) a[c] += wgt * (float)v[k][c];
+  }
+  m = mm;
+}
+
+template <bool H, int NC, bool VEC>
+__device__ __forceinline__ void merge_segments(const KParams& p, int64_t slot0, int rl, int dv, int col, int s0, int step,
+                                               int nseg, float& m, float& l, float (&a)[NC]) {
   const int64_t nrow = (int64_t)p.qrows * p.heads;
-  const int rl0 = jq * p.heads + h0;
-  const float osc = H && p.k_scale ? *p.k_scale : 1.0f;
-  for (int cb = NC * tid; cb < dv; cb += NC * 256) {
-    float m[HB], l[HB], a[HB][NC];
-#pragma unroll
-    for (int h = 0; h < HB; ++h) {
-      m[h] = kNegInf, l[h] = 0.f;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) a[h][c] = 0.f;
-    }
-    for (int s0 = 0; s0 < nseg; s0 += NS) {
-      float ls[NS][HB];
-      float v[NS][HB][NC];
-#pragma unroll
-      for (int k = 0; k < NS; ++k) {
-        const int sg = s0 + k < nseg ? s0 + k : nseg - 1;   // past the end: a valid slot, weight 0
-        const int64_t slot = (int64_t)w0 + sg + req;
-        const float* pl = p.part_lse + slot * nrow + rl0;
-#pragma unroll
-        for (int h = 0; h < HB; ++h) {
-          const int hh = h < nh ? h : 0;
-          ls[k][h] = s0 + k < nseg ? pl[hh] : kNegInf;
-          const int64_t e = (slot * nrow + rl0 + hh) * (int64_t)dv + cb;   // the slot's element
-          if constexpr (H) {
-            // fp16 partials: the slot's rows at the start of its (fp32-sized) area
-            const _Float16* src = reinterpret_cast<const _Float16*>(p.part_o + slot * nrow * (int64_t)dv) +
-                                  (e - slot * nrow * (int64_t)dv);
-            if constexpr (NC == 2) {
-              const f16x2 t = *reinterpret_cast<const f16x2*>(src);
-              v[k][h][0] = (float)t[0];
-              v[k][h][1] = (float)t[1];
-            } else {
-              const f16x8 t = *reinterpret_cast<const f16x8*>(src);
-#pragma unroll
-              for (int c = 0; c < 8; ++c) v[k][h][c] = (float)t[c];
-            }
-          } else {
-            if constexpr (NC == 2) {
-              const float2 t = *reinterpret_cast<const float2*>(p.part_o + e);
-              v[k][h][0] = t.x;
-              v[k][h][1] = t.y;
-            } else {
-              const f32x4 t0 = *reinterpret_cast<const f32x4*>(p.part_o + e);
-              const f32x4 t1 = *reinterpret_cast<const f32x4*>(p.part_o + e + 4);
-#pragma unroll
-              for (int c = 0; c < 4; ++c) {
-                v[k][h][c] = t0[c];
-                v[k][h][4 + c] = t1[c];
-              }
-            }
-          }
-        }
-      }
-#pragma unroll
-      for (int h = 0; h < HB; ++h) {
-        // segments without tokens (lse -inf) weigh 0 and a batch of them only is skipped; a NaN lse
-        // (fmaxf skips it) weighs NaN, so a row whose inputs hold a NaN merges to NaN
-        float mm = m[h];
-        bool live = false;
-#pragma unroll
-        for (int k = 0; k < NS; ++k) {
-          mm = fmaxf(mm, ls[k][h]);
-          live |= !is_neg_inf(ls[k][h]);
-        }
-        if (!live) continue;
-        const float sc = m[h] == kNegInf ? 0.f : __expf(m[h] - mm);
-        l[h] *= sc;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) a[h][c] *= sc;
-#pragma unroll
-        for (int k = 0; k < NS; ++k) {
-          const float wgt = is_neg_inf(ls[k][h]) ? 0.f : __expf(ls[k][h] - mm);
-          l[h] += wgt;
-#pragma unroll
-          for (int c = 0; c < NC; ++c) a[h][c] += wgt * v[k][h][c];
-        }
-        m[h] = mm;
-      }
-    }
-#pragma unroll
-    for (int h = 0; h < HB; ++h) {
-      if (h >= nh) continue;
-      const float inv = inv_sum(osc, l[h]);
-      const int64_t ob = (int64_t)row * p.o_sr + (int64_t)(h0 + h) * p.o_sh + cb;
-#pragma unroll
-      for (int c = 0; c < NC; ++c)
-        if (cb + c < dv) store_out(p.out, p.out_dt, ob + c, a[h][c] * inv);
-      if (cb == 0 && p.lse) store_out(p.lse, p.lse_dt, (int64_t)row * p.lse_sr + h0 + h, empty_sum(l[h]) ? kNegInf : m[h] + __logf(l[h]));
-    }
+  for (; s0 < nseg; s0 += 8 * step) {
+    const int left = (nseg - s0 + step - 1) / step;   // the same for every lane
+    if (left > 4) merge_batch<H, NC, VEC, 8>(p, slot0, nrow, rl, dv, col, s0, step, nseg, m, l, a);
+    else if (left > 2) merge_batch<H, NC, VEC, 4>(p, slot0, nrow, rl, dv, col, s0, step, nseg, m, l, a);
+    else merge_batch<H, NC, VEC, 2>(p, slot0, nrow, rl, dv, col, s0, step, nseg, m, l, a);
   }
 }
 
-// HB heads per workgroup: CH_HB, or 1 on the wide latent rows (d_c 1792 rank 1792, combine stage
-// bf16 / fp8 rows: 18.9 / 18.6 us with 2 heads, 17.4 / 16.9 with 1, 21.5 / 22.4 with 4)
-template <int HB>
-__global__ __launch_bounds__(256) void combine_bal_kernel(const KParams p, int dv) {
-  const int hblk = blockIdx.x, row = blockIdx.y;
-  const int tid = threadIdx.x;
+// H = fp16 partials without the fp8 scale, which is applied here; nch chunks of 64*NC columns per
+// row; `split` waves per chunk (1 unless SPLIT). Workgroups of nch*split waves (SPLIT: one head), or
+// of CM_AW waves that take the chunks of CM_AW / nch heads.
+template <bool H, int NC, bool SPLIT>
+__global__ __launch_bounds__(64 * (SPLIT ? CM_MW : CM_AW)) void combine_bal_kernel(const KParams p, int dv, int nch, int split) {
+  constexpr int CW = 64 * NC;
+  const int row = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int req = row / p.qrows, jq = row - req * p.qrows;
-  const int h0 = hblk * HB;
-  const int nh = p.heads - h0 < HB ? p.heads - h0 : HB;
+  // the wave's head, chunk of columns and, with SPLIT, share of the segments
+  const int hpb = SPLIT ? 1 : CM_AW / nch;
+  const int unit = SPLIT ? wv / split : wv, sub = SPLIT ? wv - unit * split : 0;
+  const int hh = SPLIT ? 0 : unit / nch, ch = SPLIT ? unit : unit - hh * nch;
+  const int head = (int)blockIdx.x * hpb + hh;
+  if (!SPLIT && (hh >= hpb || head >= p.heads)) return;
+  const float osc = H && p.k_scale ? *p.k_scale : 1.0f;
   const int chunk = p.plan[0];
   const int c0 = p.plan[2 + req], c1 = p.plan[3 + req];
+  const int64_t ob = (int64_t)row * p.o_sr + (int64_t)head * p.o_sh;
+  const int64_t lb = (int64_t)row * p.lse_sr + head;
+  const int col = ch * CW + lane * NC;
   if (c1 <= c0) {  // empty request: zero output, -inf lse
-    for (int h = 0; h < nh; ++h)
-      for (int c = tid; c < dv; c += 256)
-        store_out(p.out, p.out_dt, (int64_t)row * p.o_sr + (int64_t)(h0 + h) * p.o_sh + c, 0.f);
-    if (tid < nh && p.lse) store_out(p.lse, p.lse_dt, (int64_t)row * p.lse_sr + h0 + tid, kNegInf);
+    if (sub == 0) {
+      for (int c = 0; c < NC; ++c)
+        if (col + c < dv) store_out(p.out, p.out_dt, ob + col + c, 0.f);
+      if (ch == 0 && lane == 0 && p.lse) store_out(p.lse, p.lse_dt, lb, kNegInf);
+    }
     return;
   }
   // the first workgroup with tokens of the request holds its first token's tile (c0 + plan_sw)
   const int w0 = (c0 + p.plan_sw) / chunk, w1 = (c1 - 1) / chunk;
   if (w0 == w1) return;
   const int nseg = w1 - w0 + 1;
-  // the wide latent rows: 8 columns a thread (partials 16-byte aligned: dv % 8). Measured at d_c
-  // 1792 (combine stage, bf16 / fp8 rows): 25.4 / 23.8 us with 2 columns, 18.8 / 18.9 with 8; 8
-  // segments a batch instead of 4: 19.0 / 22.3
-  const bool w8 = dv > 1024 && dv % 8 == 0;
-  if (p.part_h) {
-    if (w8) combine_cols<true, 8, HB>(p, dv, row, jq, req, h0, nh, w0, nseg);
-    else combine_cols<true, 2, HB>(p, dv, row, jq, req, h0, nh, w0, nseg);
+  float m = kNegInf, l = 0.f, a[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) a[c] = 0.f;
+  const int lc = col < dv ? col : 0, rl = jq * p.heads + head;
+  // rows of whole lane vectors (every compiled layout), else element loads
+  if (dv % NC == 0) merge_segments<H, NC, true>(p, (int64_t)w0 + req, rl, dv, lc, sub, split, nseg, m, l, a);
+  else merge_segments<H, NC, false>(p, (int64_t)w0 + req, rl, dv, lc, sub, split, nseg, m, l, a);
+  if constexpr (!SPLIT) {
+    const float inv = inv_sum(osc, l);
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      if (col + c < dv) store_out(p.out, p.out_dt, ob + col + c, a[c] * inv);
+    if (ch == 0 && lane == 0 && p.lse) store_out(p.lse, p.lse_dt, lb, empty_sum(l) ? kNegInf : m + __logf(l));
   } else {
-    if (w8) combine_cols<false, 8, HB>(p, dv, row, jq, req, h0, nh, w0, nseg);
-    else combine_cols<false, 2, HB>(p, dv, row, jq, req, h0, nh, w0, nseg);
+    __shared__ float s_a[CM_MW][CW];
+    __shared__ float s_m[CM_MW], s_l[CM_MW];
+#pragma unroll
+    for (int q = 0; q < NC / 4; ++q)
+      *reinterpret_cast<f32x4*>(&s_a[wv][lane * NC + 4 * q]) = f32x4{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+    if (lane == 0) {
+      s_m[wv] = m;
+      s_l[wv] = l;
+    }
+    __syncthreads();
+    // a chunk's waves that had segments, their weights (the same for every chunk)
+    const int live = nseg < split ? nseg : split;
+    float wgt[CM_MW], mm = kNegInf, ll = 0.f;
+#pragma unroll
+    for (int k = 0; k < CM_MW; ++k) mm = k < live ? fmaxf(mm, s_m[k]) : mm;
+#pragma unroll
+    for (int k = 0; k < CM_MW; ++k) {
+      const float lk = s_l[k];
+      const bool on = k < live && !empty_sum(lk);
+      wgt[k] = on ? __expf(s_m[k] - mm) : 0.f;
+      ll += on ? lk * wgt[k] : 0.f;
+    }
+    const float inv = inv_sum(osc, ll);
+    for (int c = tid; c < dv; c += 64 * nch * split) {
+      const int u = c / CW;
+      float x = 0.f;
+#pragma unroll
+      for (int k = 0; k < CM_MW; ++k)
+        if (k < live) x += wgt[k] * s_a[u * split + k][c - u * CW];
+      store_out(p.out, p.out_dt, ob + c, x * inv);
+    }
+    if (tid == 0 && p.lse) store_out(p.lse, p.lse_dt, lb, empty_sum(ll) ? kNegInf : mm + __logf(ll));
   }
 }
 
@@ -1228,10 +1243,24 @@ static int run_combine(const qmla_decode_params* p, KParams& k, hipStream_t st) 
   int dv = p->d_c / p->groups;
   void* args[] = {&k, &dv};
   if (p->num_splits == 0 && (dv & 1)) return QMLA_ERR_SHAPE;   // the balanced combine reads column pairs
-  if (p->num_splits == 0)
-    return dv > 1024 ? launch((const void*)&combine_bal_kernel<1>, dim3(p->heads, p->rows, 1), dim3(256, 1, 1), args, st)
-                     : launch((const void*)&combine_bal_kernel<CH_HB>, dim3((p->heads + CH_HB - 1) / CH_HB, p->rows, 1),
-                              dim3(256, 1, 1), args, st);
+  if (p->num_splits == 0) {
+    // columns a lane and chunks of columns per (row, head); a chunk is split over up to 8 waves while
+    // they stay within 2048, 8 a CU (23 rank-768 requests, 1104 chunks: 7.9 us unsplit, 10.8 split
+    // over 4; bf16 B 4, 96 chunks: 4.3 split over 8, 7.2 unsplit)
+    const int nc = dv <= 256 ? 4 : 8;
+    int nch = (dv + 64 * nc - 1) / (64 * nc), split = 1;
+    const int64_t chunks = (int64_t)p->rows * p->heads * nch;
+    while (2 * split * nch <= CM_MW && chunks * 2 * split <= 2048) split *= 2;
+    const int hpb = split > 1 ? 1 : CM_AW / nch;
+    void* cargs[] = {&k, &dv, &nch, &split};
+    const dim3 grid((p->heads + hpb - 1) / hpb, p->rows, 1), block(64 * (split > 1 ? nch * split : CM_AW), 1, 1);
+#define QMLA_CMB(H, NC) \
+    (split > 1 ? (const void*)&combine_bal_kernel<H, NC, true> : (const void*)&combine_bal_kernel<H, NC, false>)
+    const void* fn = k.part_h ? (nc == 4 ? QMLA_CMB(true, 4) : QMLA_CMB(true, 8))
+                              : (nc == 4 ? QMLA_CMB(false, 4) : QMLA_CMB(false, 8));
+#undef QMLA_CMB
+    return launch(fn, grid, block, cargs, st);
+  }
   return launch((const void*)&combine_kernel, dim3(p->heads, p->rows, 1), dim3(256, 1, 1), args, st);
 }
 
