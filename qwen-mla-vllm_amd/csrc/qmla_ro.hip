@@ -134,7 +134,7 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
   const float lc2 = 3.0f + fast_log2(c2b != 0.f ? fabsf(c2b) : 1.0f);
   const float qsign = c2b > 0.f ? 1.0f : c2b < 0.f ? -1.0f : 0.0f;
   float mref = kNegInf, lpart = 0.f;
-  f32x4 acc[ROLE == COMPUTE ? C::CB : 1];
+  f32x4 acc[ROLE == COMPUTE ? C::CB : 1];   // columns 16cb + 4lg + i of row rg
 #pragma unroll
   for (int cb = 0; cb < (ROLE == COMPUTE ? C::CB : 1); ++cb) acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
@@ -197,45 +197,12 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
     for (int e = 0; e < 8; ++e) qh8[C::NB][e] = lg < 2 ? hq[8 * C::NB + e] : lq[8 * C::NB + e];
   };
 
-  // normalize and write the rows of request req (accumulator row 16rbk + 4lg + i on this lane)
+  // normalize and write the rows of request req (row rg on this lane)
   auto finalize = [&](int req, int fl) {
-    const SegOut so = seg_out<C::DCG>(p, req, (fl & SEG_FINAL) != 0, wr);
+    const RowOut o = row_out<C::DCG>(p, seg_out<C::DCG>(p, req, (fl & SEG_FINAL) != 0, wr), req * qrows, kscale);
     const float l = sum_lg(lpart);
-    const float inv = inv_sum(kscale, l);   // fp8 values were accumulated unscaled
-    const float invh = inv_sum(1.0f, l);    // ... and are stored so as fp16 partials
-    const float lse_v = row_lse(mref, l);
-    const int row0 = req * qrows;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float inv_i = __shfl(inv, 4 * lg + i, 64);   // row 4lg+i's values sit on lane 4lg+i
-      const int ri = 16 * rbk + 4 * lg + i;
-      if (ri >= nrows) continue;
-      const int jr = ri % qrows, h = grp * hpg + ri / qrows;
-      const int col = ln16;
-      if (so.final_out) {
-        const int64_t ob = (int64_t)(row0 + jr) * p.o_sr + (int64_t)h * p.o_sh + col;
-#pragma unroll
-        for (int cb = 0; cb < C::CB; ++cb) store_out(p.out, p.out_dt, ob + 16 * cb, acc[cb][i] * inv_i);
-      } else if (so.plse && p.part_h) {
-        _Float16* ob = reinterpret_cast<_Float16*>(so.po) + (int64_t)jr * so.po_sr + (int64_t)h * so.po_sh + col;
-        const float invh_i = __shfl(invh, 4 * lg + i, 64);
-#pragma unroll
-        for (int cb = 0; cb < C::CB; ++cb) ob[16 * cb] = (_Float16)(acc[cb][i] * invh_i);
-      } else {
-        float* ob = so.po + (int64_t)jr * so.po_sr + (int64_t)h * so.po_sh + col;
-#pragma unroll
-        for (int cb = 0; cb < C::CB; ++cb) ob[16 * cb] = acc[cb][i] * inv_i;
-      }
-    }
-    if (lg == 0 && rok) {
-      if (so.final_out) {
-        if (p.lse) store_out(p.lse, p.lse_dt, (int64_t)(row0 + jq) * p.lse_sr + head, lse_v);
-      } else if (so.plse) {
-        so.plse[(int64_t)jq * so.plse_sr + head] = lse_v;
-      } else {
-        so.po[(int64_t)jq * so.po_sr + (int64_t)head * so.po_sh + C::DCG] = lse_v;
-      }
-    }
+    if (lg == 0 && rok && o.lse) store_out(o.lse, o.lse_dt, jq * o.lse_sr + head * o.lse_sh, row_lse(mref, l));
+    store_row(o, acc, inv_sum(o.num, l), jq * o.sr + head * o.sh, rok);
   };
 
   // ---- DMA wave: instruction i = dw + 2j covers LDS chunks 64i .. 64i+63 of a stage (staged row
@@ -555,11 +522,7 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
             mref = mn;
             lpart *= al;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const float a_i = __shfl(al, 4 * lg + i, 64);   // accumulator row 4lg+i
-#pragma unroll
-              for (int c = 0; c < C::CB; ++c) acc[c][i] *= a_i;
-            }
+            for (int c = 0; c < C::CB; ++c) acc[c] *= al;
           }
           const float mu = mref == kNegInf ? 0.f : mref;
           f16x8 pf;
@@ -577,7 +540,7 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
           static_for<0, C::CB>([&](auto cc) {
             constexpr int c = decltype(cc)::value;
             lds_wait_n<cmin15(C::CB - 1 - c)>(vraw[c]);
-            acc[c] = mfma16(pf, __builtin_bit_cast(f16x8, vraw[c]), acc[c]);
+            acc[c] = mfma16(__builtin_bit_cast(f16x8, vraw[c]), pf, acc[c]);
           });
         }
         if (++ts == s_nt) {

@@ -59,6 +59,11 @@ __device__ __forceinline__ void ldsr32f3_drained(const void* a, const void* b, c
       : "v"(lds_addr(static_cast<const char*>(a))), "v"(lds_addr(static_cast<const char*>(b))),
         "v"(lds_addr(static_cast<const char*>(c))));
 }
+__device__ __forceinline__ void ldsr32f2_drained(const void* a, const void* b, float& x, float& y) {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\tds_read_b32 %0, %2\n\tds_read_b32 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+               : "=&v"(x), "=&v"(y)
+               : "v"(lds_addr(static_cast<const char*>(a))), "v"(lds_addr(static_cast<const char*>(b))));
+}
 __device__ __forceinline__ void ldsr128x2_drained(const void* a, const void* b, i32x4& x, i32x4& y) {
   asm volatile("s_waitcnt lgkmcnt(0)\n\tds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
                : "=&v"(x), "=&v"(y)

@@ -271,7 +271,7 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
     }
   };
 
-  // ---- value wave: accumulator of the group's rows (16mb + 4lg + i) x its columns VC*vh + 16cb + ln16 ----
+  // ---- value wave: accumulator of the group's rows 16mb + ln16 x its columns VC*vh + 16cb + 4lg + i ----
   f32x4 acc[C::MBV][ROLE == VALUE ? C::CB : 1];
   auto zero_acc = [&]() {
 #pragma unroll
@@ -361,53 +361,23 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
     }
   };
   // value wave: normalize and write the output of request req, whose sums are in fin[k & 1]
+  const uint32_t hpw_inv = (65536u + hpw - 1) / hpw;   // row / hpw = (row * hpw_inv) >> 16 for rows < 128
   auto finalize = [&](int k, int req, int fl) {
-    const SegOut so = seg_out<C::DCG>(p, req, (fl & SEG_FINAL) != 0, wr);
-    const int row0 = req * qrows;
+    const RowOut o = row_out<C::DCG>(p, seg_out<C::DCG>(p, req, (fl & SEG_FINAL) != 0, wr), req * qrows, kscale);
+    int ln = lane;
+    asm volatile("" : "+v"(ln));   // the row offsets are computed here, not kept across the tile loop
+    const int l16 = ln & 15, g4 = ln >> 4;
 #pragma unroll
-    for (int mb = 0; mb < C::MBV; ++mb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int rr = 16 * mb + 4 * lg + i;        // row within the group
-        const int rw = 16 * C::MBV * vg + rr;       // row of the workgroup's arrays
-        float m, l0, l1;
-        if constexpr (C::G == 1) {
-          m = ldsr32f(&sm.fin[k & 1][0][0][rw]);
-          l0 = ldsr32f(&sm.fin[k & 1][1][0][rw]);
-          l1 = ldsr32f(&sm.fin[k & 1][1][1][rw]);
-          lds_wait_n<2>(m);
-          lds_wait_n<1>(l0);
-          lds_wait_n<0>(l1);
-        } else {
-          ldsr32f3_drained(&sm.fin[k & 1][0][0][rw], &sm.fin[k & 1][1][0][rw], &sm.fin[k & 1][1][1][rw], m, l0, l1);
-        }
-        if (rr >= nrows) continue;
-        const float l = l0 + l1;
-        const int jr = rr / hpw, h = vg * hpg + h0 + rr - jr * hpw;
-        const float inv = inv_sum(kscale, l);   // fp8 values were accumulated unscaled
-        const float lse_v = row_lse(m, l);
-        const int col = C::VC * vh + ln16;
-        if (so.final_out) {
-          const int64_t ob = (int64_t)(row0 + jr) * p.o_sr + (int64_t)h * p.o_sh + col;
-#pragma unroll
-          for (int cb = 0; cb < C::CB; ++cb) store_out(p.out, p.out_dt, ob + 16 * cb, acc[mb][cb][i] * inv);
-          if (vh == 0 && ln16 == 0 && p.lse) store_out(p.lse, p.lse_dt, (int64_t)(row0 + jr) * p.lse_sr + h, lse_v);
-        } else if (so.plse && p.part_h) {
-          _Float16* ob = reinterpret_cast<_Float16*>(so.po) + (int64_t)jr * so.po_sr + (int64_t)h * so.po_sh + col;
-          const float invh = inv_sum(1.0f, l);
-#pragma unroll
-          for (int cb = 0; cb < C::CB; ++cb) ob[16 * cb] = (_Float16)(acc[mb][cb][i] * invh);
-          if (vh == 0 && ln16 == 0) so.plse[(int64_t)jr * so.plse_sr + h] = lse_v;
-        } else {
-          float* ob = so.po + (int64_t)jr * so.po_sr + (int64_t)h * so.po_sh + col;
-#pragma unroll
-          for (int cb = 0; cb < C::CB; ++cb) ob[16 * cb] = acc[mb][cb][i] * inv;
-          if (vh == 0 && ln16 == 0) {
-            if (so.plse) so.plse[(int64_t)jr * so.plse_sr + h] = lse_v;
-            else so.po[(int64_t)jr * so.po_sr + (int64_t)h * so.po_sh + C::DCG] = lse_v;
-          }
-        }
-      }
+    for (int mb = 0; mb < C::MBV; ++mb) {
+      const int rr = 16 * mb + l16;                      // row within the group
+      const int rw = 16 * C::MBV * vg + rr;              // row of the workgroup's arrays
+      float m, l0, l1;
+      ldsr32f3_drained(&sm.fin[k & 1][0][0][rw], &sm.fin[k & 1][1][0][rw], &sm.fin[k & 1][1][1][rw], m, l0, l1);
+      const float l = l0 + l1;
+      const int jr = (int)((rr * hpw_inv) >> 16), h = vg * hpg + h0 + rr - jr * hpw;
+      if (vh == 0 && g4 == 0 && rr < nrows && o.lse) store_out(o.lse, o.lse_dt, jr * o.lse_sr + h * o.lse_sh, row_lse(m, l));
+      store_row(o, acc[mb], inv_sum(o.num, l), jr * o.sr + h * o.sh + C::VC * vh, rr < nrows);
+    }
     zero_acc();
   };
 
@@ -843,19 +813,16 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
           for (int mb = 0; mb < C::MBV; ++mb) fany |= fm[mb];
           if (fany) {
             // the reference of some row moved at tile j: rescale before adding it
-            i32x4 ar[C::MBV];
+            float al[C::MBV];
 #pragma unroll
-            for (int mb = 0; mb < C::MBV; ++mb) ar[mb] = ldsr128(&sm.alpha[pj][vr0 + 16 * mb + 4 * lg]);
+            for (int mb = 0; mb < C::MBV; ++mb) al[mb] = ldsr32f(&sm.alpha[pj][vr0 + 16 * mb + ln16]);
 #pragma unroll
-            for (int mb = 0; mb < C::MBV; ++mb) lds_wait_n<0>(ar[mb]);
+            for (int mb = 0; mb < C::MBV; ++mb) lds_wait_n<0>(al[mb]);
 #pragma unroll
             for (int mb = 0; mb < C::MBV; ++mb) {
               if (fm[mb] == 0) continue;
-              const f32x4 al = __builtin_bit_cast(f32x4, ar[mb]);
 #pragma unroll
-              for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int cb = 0; cb < C::CB; ++cb) acc[mb][cb][i] *= al[i];
+              for (int cb = 0; cb < C::CB; ++cb) acc[mb][cb] *= al[mb];
             }
           }
           using PX8 = typename C::PX8;
@@ -878,7 +845,7 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
               vf = __builtin_bit_cast(PX8, w4);
             }
 #pragma unroll
-            for (int mb = 0; mb < C::MBV; ++mb) acc[mb][cb] = mfma16(pf[mb], vf, acc[mb][cb]);
+            for (int mb = 0; mb < C::MBV; ++mb) acc[mb][cb] = mfma16(vf, pf[mb], acc[mb][cb]);
           });
           if (++tv == v_nt) {
             // the request's last tile: its sums were published at the previous step

@@ -248,7 +248,7 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
   float mref = kNegInf, lpart = 0.f;   // the row's reference max (log2 domain) and partial sum
   int lim = 0;                          // the row's token limit in the current piece
 
-  // ---- value wave: accumulator of rows 16mb + 4lg + i x columns VC*vw + 16cb + ln16 ----
+  // ---- value wave: accumulator of rows 16mb + ln16 x columns VC*vw + 16cb + 4lg + i ----
   f32x4 acc[2][QS ? 1 : C::CB];
   auto zero_acc = [&]() {
 #pragma unroll
@@ -321,44 +321,20 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
   };
 
   // value wave: normalize and write the output of request req, whose sums are in fin[k & 1]
+  const uint32_t hpw_inv = (65536u + hpw - 1) / hpw;   // row / hpw = (row * hpw_inv) >> 16 for rows < 32
   auto finalize = [&](int k, int req, int fl) {
-    const SegOut so = seg_out<C::DC>(p, req, (fl & SEG_FINAL) != 0, wr);
-    const int row0 = req * qrows;
+    const RowOut o = row_out<C::DC>(p, seg_out<C::DC>(p, req, (fl & SEG_FINAL) != 0, wr), req * qrows, kscale);
+    int ln = lane;
+    asm volatile("" : "+v"(ln));   // the row offsets are computed here, not kept across the tile loop
+    const int l16 = ln & 15, g4 = ln >> 4;
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb) {
-      i32x4 mr, lr;
-      ldsr128x2_drained(&sm.fin[k & 1][0][16 * mb + 4 * lg], &sm.fin[k & 1][1][16 * mb + 4 * lg], mr, lr);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int rr = 16 * mb + 4 * lg + i;
-        if (rr >= nrows) continue;
-        const float m = __int_as_float(mr[i]), l = __int_as_float(lr[i]);
-        const int jr = rr / hpw, h = h0 + rr - jr * hpw;
-        const float inv = inv_sum(kscale, l);   // fp8 values were accumulated unscaled
-        const float lse_v = row_lse(m, l);
-        const int col = C::VC * vw + ln16;
-        if (so.final_out) {
-          const int64_t ob = (int64_t)(row0 + jr) * p.o_sr + (int64_t)h * p.o_sh + col;
-#pragma unroll
-          for (int cb = 0; cb < C::CB; ++cb) store_out(p.out, p.out_dt, ob + 16 * cb, acc[mb][cb][i] * inv);
-          if (vw == 0 && ln16 == 0 && p.lse) store_out(p.lse, p.lse_dt, (int64_t)(row0 + jr) * p.lse_sr + h, lse_v);
-        } else if (so.plse && p.part_h) {
-          // fp16 partials without the fp8 scale, which the combine applies
-          _Float16* ob = reinterpret_cast<_Float16*>(so.po) + (int64_t)jr * so.po_sr + (int64_t)h * so.po_sh + col;
-          const float invh = inv_sum(1.0f, l);
-#pragma unroll
-          for (int cb = 0; cb < C::CB; ++cb) ob[16 * cb] = (_Float16)(acc[mb][cb][i] * invh);
-          if (vw == 0 && ln16 == 0) so.plse[(int64_t)jr * so.plse_sr + h] = lse_v;
-        } else {
-          float* ob = so.po + (int64_t)jr * so.po_sr + (int64_t)h * so.po_sh + col;
-#pragma unroll
-          for (int cb = 0; cb < C::CB; ++cb) ob[16 * cb] = acc[mb][cb][i] * inv;
-          if (vw == 0 && ln16 == 0) {
-            if (so.plse) so.plse[(int64_t)jr * so.plse_sr + h] = lse_v;
-            else so.po[(int64_t)jr * so.po_sr + (int64_t)h * so.po_sh + C::DC] = lse_v;
-          }
-        }
-      }
+      const int rr = 16 * mb + l16;
+      float m, l;
+      ldsr32f2_drained(&sm.fin[k & 1][0][rr], &sm.fin[k & 1][1][rr], m, l);
+      const int jr = (int)((rr * hpw_inv) >> 16), h = h0 + rr - jr * hpw;
+      if (vw == 0 && g4 == 0 && rr < nrows && o.lse) store_out(o.lse, o.lse_dt, jr * o.lse_sr + h * o.lse_sh, row_lse(m, l));
+      store_row(o, acc[mb], inv_sum(o.num, l), jr * o.sr + h * o.sh + C::VC * vw, rr < nrows);
     }
     zero_acc();
   };
@@ -689,19 +665,16 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
           const int f0 = __builtin_amdgcn_readfirstlane(flw[0]), f1 = __builtin_amdgcn_readfirstlane(flw[1]);
           if (f0 | f1) {
             // some row's reference moved at tile j: rescale before adding it
-            i32x4 ar[2];
+            float al[2];
 #pragma unroll
-            for (int mb = 0; mb < 2; ++mb) ar[mb] = ldsr128(&sm.alpha[pj][16 * mb + 4 * lg]);
+            for (int mb = 0; mb < 2; ++mb) al[mb] = ldsr32f(&sm.alpha[pj][16 * mb + ln16]);
 #pragma unroll
-            for (int mb = 0; mb < 2; ++mb) lds_wait_n<0>(ar[mb]);
+            for (int mb = 0; mb < 2; ++mb) lds_wait_n<0>(al[mb]);
 #pragma unroll
             for (int mb = 0; mb < 2; ++mb) {
               if ((mb == 0 ? f0 : f1) == 0) continue;
-              const f32x4 al = __builtin_bit_cast(f32x4, ar[mb]);
 #pragma unroll
-              for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int cb = 0; cb < C::CB; ++cb) acc[mb][cb][i] *= al[i];
+              for (int cb = 0; cb < C::CB; ++cb) acc[mb][cb] *= al[mb];
             }
           }
           using PX8 = typename C::PX8;
@@ -723,7 +696,7 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
               vf = __builtin_bit_cast(PX8, w4);
             }
 #pragma unroll
-            for (int mb = 0; mb < 2; ++mb) acc[mb][c] = mfma16(pf[mb], vf, acc[mb][c]);
+            for (int mb = 0; mb < 2; ++mb) acc[mb][c] = mfma16(vf, pf[mb], acc[mb][c]);
           });
           if (++tv == v_nt) {
             // the request's last tile: its sums were published with it
