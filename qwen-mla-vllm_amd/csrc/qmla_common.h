@@ -26,6 +26,8 @@ struct KParams {
   const char* kv;
   int64_t page_stride_b, token_stride_b;  // bytes
   int page_size;
+  uint32_t page_mul;    // x / page_size = (x * page_mul) >> page_sh for 0 <= x < 2^31 (page_magic)
+  int page_sh;
   int rope_w;
   int rms_off_b;  // byte offset of the rms tail inside a row
   const float* k_scale;
@@ -61,6 +63,18 @@ struct KParams {
   int part_h;           // balanced partial outputs in fp16 and without the fp8 scale (fp8 caches:
                         // |value| <= 448), which the combine applies; else fp32
 };
+
+// x / d = (x * mul) >> sh for 0 <= x < 2^31: sh = 31 + ceil(log2 d), mul = ceil(2^sh / d) < 2^32, so
+// mul exceeds 2^sh / d by less than one part in 2^31 * d / 2^sh.
+inline void page_magic(int d, uint32_t& mul, int& sh) {
+  int l = 0;
+  while (((int64_t)1 << l) < d) ++l;
+  sh = 31 + l;
+  mul = (uint32_t)((((uint64_t)1 << sh) + (uint64_t)d - 1) / (uint64_t)d);
+}
+__device__ __forceinline__ int page_div(const KParams& p, int x) {
+  return (int)(((uint64_t)(uint32_t)x * p.page_mul) >> p.page_sh);
+}
 
 // A block-table entry checked against the page bound: an entry outside [0, page_bound) reads page 0
 // (in bounds) and raises `bad`, which the kernel reports once its memory traffic has drained.
@@ -117,20 +131,26 @@ __device__ __forceinline__ int req_len(const KParams& p, int req) {
 // than the scan, and inside a HIP graph far more), and workgroup 0 also stores the plan for the
 // balanced combine.
 
+// inclusive prefix sums over the 64 lanes, all of them active: DPP row shifts inside each 16 lanes,
+// then the last lane of a row added to the rows after it
 __device__ __forceinline__ int wave_incl_sum(int x) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);   // row_shr 1, 2, 4, 8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);   // row_bcast 15 into rows 1, 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);   // row_bcast 31 into rows 2, 3
   return x;
 }
+__device__ __forceinline__ int lane_value(int x, int lane) { return __builtin_amdgcn_readlane(x, lane); }
 
 template <int SW>
-__device__ __forceinline__ int plan_tiles(const KParams& p, int b) {
-  const int L = req_len(p, b);
+__device__ __forceinline__ int len_tiles(int L) {
   return L > 0 ? (L + PLAN_TILE - 1) / PLAN_TILE + SW : 0;
+}
+template <int SW>
+__device__ __forceinline__ int plan_tiles(const KParams& p, int b) {
+  return len_tiles<SW>(req_len(p, b));
 }
 
 // The tokens [a, e) of a request of length L with plan tiles [c0, c1) that plan tiles [lo, hi) hold
@@ -156,41 +176,63 @@ struct BalRange {
   int b0, c0;      // the last request with C_b <= lo, and its C_b
 };
 
-// One wave computes workgroup w's range (wave-uniform results; any wave may call it).
+// One wave computes workgroup w's range (wave-uniform results; any wave may call it). The lengths of
+// the first 256 requests are loaded at once and kept for the second pass; with a load and a scan over
+// LDS permutes per 64 requests in each pass, range and window took 3.5 us at a workgroup's start, 2.4
+// now, with the page divisions by multiplication (one request of 1300 tokens).
 template <int SW>
 __device__ inline BalRange balanced_range(const KParams& p, int w) {
+  constexpr int NK = 4;
   const int lane = threadIdx.x & 63;
   BalRange r;
-  int total = 0;
-  for (int base = 0; base < p.n_req; base += 64) {
-    const int b = base + lane;
-    total += __shfl(wave_incl_sum(b < p.n_req ? plan_tiles<SW>(p, b) : 0), 63, 64);
+  r.chunk = 1;
+  r.lo = r.hi = r.total = r.b0 = r.c0 = 0;
+  if (p.n_req <= 0) return r;
+  int t[NK], incl[NK];
+#pragma unroll
+  for (int k = 0; k < NK; ++k) {
+    const int b = 64 * k + lane;
+    t[k] = req_len(p, b < p.n_req ? b : p.n_req - 1);
   }
-  // wave-uniform values: scalar registers (shuffle results are vector registers to the compiler)
-  total = __builtin_amdgcn_readfirstlane(total);
+  int total = 0;
+#pragma unroll
+  for (int k = 0; k < NK; ++k) {
+    t[k] = 64 * k + lane < p.n_req ? len_tiles<SW>(t[k]) : 0;
+    incl[k] = wave_incl_sum(t[k]);
+    total += lane_value(incl[k], 63);
+  }
+  for (int base = 64 * NK; base < p.n_req; base += 64) {
+    const int b = base + lane;
+    total += lane_value(wave_incl_sum(b < p.n_req ? plan_tiles<SW>(p, b) : 0), 63);
+  }
   r.total = total;
   r.chunk = total > 0 ? (total + p.nwg - 1) / p.nwg : 1;
   r.lo = w * r.chunk;
   r.hi = r.lo + r.chunk < total ? r.lo + r.chunk : total;
-  r.b0 = 0;
-  r.c0 = 0;
   if (r.lo >= r.hi) return r;
-  int run = 0;
-  for (int base = 0; base < p.n_req && run <= r.lo; base += 64) {
-    const int b = base + lane;
-    const int t = b < p.n_req ? plan_tiles<SW>(p, b) : 0;
-    const int incl = wave_incl_sum(t);
-    const int c = run + incl - t;
-    const uint64_t m = __builtin_amdgcn_ballot_w64(b < p.n_req && c <= r.lo);
+  // the last request with C_b <= lo among 64 requests from base, whose tiles start at `run`
+  auto find = [&](int base, int run, int tiles, int in) {
+    const int c = run + in - tiles;
+    const uint64_t m = __builtin_amdgcn_ballot_w64(base + lane < p.n_req && c <= r.lo);
     if (m) {
       const int x = 63 - __builtin_clzll(m);
       r.b0 = base + x;
-      r.c0 = __shfl(c, x, 64);
+      r.c0 = lane_value(c, x);
     }
-    run += __shfl(incl, 63, 64);
+  };
+  int run = 0;
+#pragma unroll
+  for (int k = 0; k < NK; ++k) {
+    find(64 * k, run, t[k], incl[k]);
+    run += lane_value(incl[k], 63);
   }
-  r.b0 = __builtin_amdgcn_readfirstlane(r.b0);
-  r.c0 = __builtin_amdgcn_readfirstlane(r.c0);
+  for (int base = 64 * NK; base < p.n_req && run <= r.lo; base += 64) {
+    const int b = base + lane;
+    const int tb = b < p.n_req ? plan_tiles<SW>(p, b) : 0;
+    const int in = wave_incl_sum(tb);
+    find(base, run, tb, in);
+    run += lane_value(in, 63);
+  }
   return r;
 }
 
@@ -205,7 +247,7 @@ __device__ inline void store_plan(const KParams& p) {
     const int t = b < p.n_req ? plan_tiles<SW>(p, b) : 0;
     const int incl = wave_incl_sum(t);
     if (b <= p.n_req) p.plan[2 + b] = run + incl - t;
-    run += __shfl(incl, 63, 64);
+    run += lane_value(incl, 63);
   }
   if (lane == 0) {
     p.plan[0] = run > 0 ? (run + p.nwg - 1) / p.nwg : 1;

@@ -461,8 +461,8 @@ __device__ __forceinline__ void segment(const KParams& p, Smem<C>& sm, int req, 
   const bool uni = (P % C::TT) == 0 && (ta % C::TT) == 0;   // every tile within one page
   for (int sa = ta; sa < te; sa += sub) {
     const int se = te - sa < sub ? te : sa + sub;
-    const int pbase = sa / P;
-    const int np = (se - 1) / P - pbase + 1;
+    const int pbase = page_div(p, sa);
+    const int np = page_div(p, se - 1) - pbase + 1;
     wait_vmcnt<0>();
     lds_barrier();   // every wave is done with the previous sub-range's page ids
     for (int i = tid; i < np; i += C::NTHR) sm.pid[i] = checked_page(p, btrow[pbase + i], bad);
@@ -477,8 +477,8 @@ __device__ __forceinline__ void segment(const KParams& p, Smem<C>& sm, int req, 
       int ln = lane;
       asm volatile("" : "+v"(ln));   // keep the offsets from being hoisted out of the tile loop
       if (uni) {
-        const int pg = __builtin_amdgcn_readfirstlane(sm.pid[tok0 / P - pbase]);
-        const char* base = p.kv + (int64_t)pg * PS + (int64_t)(tok0 % P) * TS;
+        const int pg = __builtin_amdgcn_readfirstlane(sm.pid[page_div(p, tok0) - pbase]);
+        const char* base = p.kv + (int64_t)pg * PS + (int64_t)(tok0 - page_div(p, tok0) * P) * TS;
         // rows past the range end read as zeros (outside the resource)
         const __amdgpu_buffer_rsrc_t rs = make_rsrc(base, (uint32_t)(nvalid * TS));
         const int tb0 = tg * C::T;
@@ -539,7 +539,7 @@ __device__ __forceinline__ void segment(const KParams& p, Smem<C>& sm, int req, 
           if (CPI * k + CPI <= C::NCH || CPI * k + cl < C::NCH) {
             const int rr = row < nv ? row : (nv > 0 ? nv - 1 : 0);
             const int tok = nv > 0 ? tb0 + rr : se - 1;
-            const int q = tok / P;
+            const int q = page_div(p, tok);
             const int pg = sm.pid[q - pbase];
             const char* src = p.kv + (int64_t)pg * PS + (int64_t)(tok - q * P) * TS + off;
             if constexpr (C::DW) dma4(src, dst + k * 256);
@@ -556,7 +556,7 @@ __device__ __forceinline__ void segment(const KParams& p, Smem<C>& sm, int req, 
             if ((CPI * k + CPI <= C::T * C::CRM || j < C::T * C::CRM) && (!C::DW || ob < (int)TS)) {
               const int rr = row < nv ? row : (nv > 0 ? nv - 1 : 0);
               const int tok = nv > 0 ? tb0 + rr : se - 1;
-              const int q = tok / P;
+              const int q = page_div(p, tok);
               const int pg = sm.pid[q - pbase];
               const char* src = p.kv + (int64_t)pg * PS + (int64_t)(tok - q * P) * TS + ob;
               if constexpr (C::DW) dma4(src, rdst + k * 256);

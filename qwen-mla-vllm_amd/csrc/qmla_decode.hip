@@ -188,17 +188,17 @@ __device__ __forceinline__ void process_segment(const KParams& p, Smem<C>& sm, i
   auto issue_pid = [&](int t) {
     int tok = tok_a + t * TILE + lane;
     tok = tok < tok_e ? tok : tok_e - 1;
-    if (lane < TILE) dma4(bt + tok / P, reinterpret_cast<char*>(sm.pid[t % (2 * C::S)]));
+    if (lane < TILE) dma4(bt + page_div(p, tok), reinterpret_cast<char*>(sm.pid[t % (2 * C::S)]));
   };
   auto issue_data = [&](int t) {
     const int tok0 = tok_a + t * TILE;
     const int* pidt = sm.pid[t % (2 * C::S)];
     char* dst = sm.kv[t % C::S];
-    if (!C::DW && tok0 / P == (tok0 + TILE - 1) / P && p.token_stride_b == C::RB) {
+    if (!C::DW && page_div(p, tok0) == page_div(p, tok0 + TILE - 1) && p.token_stride_b == C::RB) {
       // the TILE rows are consecutive in one page: one contiguous block, addressed through a
       // buffer resource so the per-tile cost is scalar (rows past tok_e stay inside the page)
       const int page = checked_page(p, __builtin_amdgcn_readfirstlane(pidt[0]), bad);
-      const char* base = p.kv + (int64_t)page * p.page_stride_b + (int64_t)(tok0 % P) * p.token_stride_b;
+      const char* base = p.kv + (int64_t)page * p.page_stride_b + (int64_t)(tok0 - page_div(p, tok0) * P) * p.token_stride_b;
       const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(base, (uint32_t)(TILE * C::RB));
 #pragma unroll
       for (int j = 0; j < C::NDMA; ++j) {
@@ -210,7 +210,7 @@ __device__ __forceinline__ void process_segment(const KParams& p, Smem<C>& sm, i
     int tok = tok0 + (lane < TILE ? lane : TILE - 1);
     tok = tok < tok_e ? tok : tok_e - 1;
     const int64_t off = (int64_t)checked_page(p, pidt[lane < TILE ? lane : TILE - 1], bad) * p.page_stride_b +
-                        (int64_t)(tok % P) * p.token_stride_b;
+                        (int64_t)(tok - page_div(p, tok) * P) * p.token_stride_b;
     const int off_lo = (int)(uint32_t)off, off_hi = (int)(uint32_t)((uint64_t)off >> 32);
     if constexpr (C::DW) {
       // instruction i's 64 chunks as four 16-chunk quarters: lane l of quarter s carries the 4 bytes
@@ -1161,6 +1161,7 @@ static KParams make_kparams(const qmla_decode_params* p) {
   k.page_stride_b = p->page_stride * eb;
   k.token_stride_b = p->token_stride * eb;
   k.page_size = p->page_size;
+  page_magic(p->page_size, k.page_mul, k.page_sh);
   k.rope_w = p->rope_w;
   k.rms_off_b = p->rms_offset >= 0 ? p->rms_offset * eb : 0;
   k.k_scale = p->k_scale;

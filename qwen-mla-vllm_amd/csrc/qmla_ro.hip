@@ -270,7 +270,7 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
       }
       const SegD& d = sm.seg[k0];
       // a folded request reads the block-table row of its last verify row, as its length does
-      sm.pid[f] = checked_page(p, p.bt[((int64_t)d.req * qrows + qrows - 1) * p.bt_stride + d.ta / P + (f - d.pf)],
+      sm.pid[f] = checked_page(p, p.bt[((int64_t)d.req * qrows + qrows - 1) * p.bt_stride + page_div(p, d.ta) + (f - d.pf)],
                                bad);
     }
     __syncthreads();
@@ -285,7 +285,7 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
         i_nt = d.nt;
         i_pf = d.pf;
         ipg = d.pf;
-        ioff = d.ta % P;
+        ioff = d.ta - page_div(p, d.ta) * P;
       };
       // issues tile g into ring stage g % S and advances the cursor
       auto issue = [&](int g) {
@@ -308,8 +308,8 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
             if (drow[j] >= 0) {
               const int rr = drow[j] < nvalid ? drow[j] : nvalid - 1;
               const int tok = tok0 + rr;
-              const int q = tok / P;
-              int pg = ldsr32(&sm.pid[i_pf + q - i_ta / P]);
+              const int q = page_div(p, tok);
+              int pg = ldsr32(&sm.pid[i_pf + q - page_div(p, i_ta)]);
               lds_wait_n<0>(pg);
               const uint32_t cbo = doff[j] - (uint32_t)(drow[j] * C::RB);
               dma16(p.kv + (int64_t)pg * p.page_stride_b + (int64_t)(tok - q * P) * p.token_stride_b + cbo,

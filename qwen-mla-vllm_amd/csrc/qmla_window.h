@@ -237,18 +237,19 @@ __device__ void plan_window(const KParams& p, SM& sm, bool fixed, int lo, int hi
       }
     }
     const bool live = !beyond && a < e;
-    const int pages = live ? (e - 1) / P - a / P + 1 : 0;
+    const int pa = page_div(p, a);
+    const int pages = live ? page_div(p, e - 1) - pa + 1 : 0;
     const int cum = wave_incl_sum(pages);
     const int excl = cum - pages;
     const bool take = live && excl < PN;
     int et = e;
     if (take && cum > PN) {
-      const int cut = (a / P + (PN - excl)) * P;   // page-aligned, > a
+      const int cut = (pa + (PN - excl)) * P;   // page-aligned, > a
       et = cut < e ? cut : e;
     }
     if (et < e) fl &= ~SEG_LAST;
     const int nt = take ? (et - a + TILE - 1) / TILE : 0;
-    const int npt = take ? (et - 1) / P - a / P + 1 : 0;
+    const int npt = take ? page_div(p, et - 1) - pa + 1 : 0;
     const uint64_t tm = __builtin_amdgcn_ballot_w64(take);
     const int tcum = wave_incl_sum(nt);
     const int pcum = wave_incl_sum(npt);
@@ -265,24 +266,24 @@ __device__ void plan_window(const KParams& p, SM& sm, bool fixed, int lo, int hi
       sm.seg[lanes_below(tm)] = d;
     }
     nseg = __builtin_popcountll(tm);
-    ntot = __shfl(tcum, 63, 64);
-    npg = __shfl(pcum, 63, 64);
+    ntot = lane_value(tcum, 63);
+    npg = lane_value(pcum, 63);
     // cursor: the first live request not finished here; else the range is done if a request at or
     // past its end was seen; else the next 64 requests
     const uint64_t um = __builtin_amdgcn_ballot_w64(live && (!take || et < e));
     const uint64_t bm = __builtin_amdgcn_ballot_w64(beyond);
     if (um) {
       const int x = __builtin_ctzll(um);
-      const int etx = __shfl(et, x, 64);
+      const int etx = lane_value(et, x);
       const bool tookx = (tm >> x) & 1;
       cb += x;
-      cp = __shfl(c0, x, 64);
+      cp = lane_value(c0, x);
       ctok = tookx ? etx : 0;
     } else if (bm) {
       more = false;
     } else {
       cb += 64;
-      cp = __shfl(c1, 63, 64);
+      cp = lane_value(c1, 63);
       ctok = 0;
     }
   }
