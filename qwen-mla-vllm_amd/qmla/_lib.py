@@ -231,6 +231,33 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+def stream() -> int:
+    """The current device's current stream, as the C ABI takes it. torch.cuda.current_stream() builds
+    a Stream object for the same answer: 2.7 us a call against 0.2."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
+def keep_alive(tensors) -> None:
+    """Tell the allocator that the current stream reads these tensors (a caller's tensor may belong to
+    another stream, a converted copy dies with the call that launched its reader)."""
+    sid, index, kind = torch._C._cuda_getCurrentStream(torch.cuda.current_device())
+    s = torch.Stream(stream_id=sid, device_index=index, device_type=kind)
+    for t in tensors:
+        t.record_stream(s)
+
+
+def rows2d(t: torch.Tensor) -> torch.Tensor:
+    """[rows, the rest flattened]: the tensor itself where it is that already."""
+    return t if t.dim() == 2 and t.numel() > 0 else t.reshape(t.shape[0], -1)
+
+
+def as_scale(t: torch.Tensor, device) -> torch.Tensor:
+    """A scale's first element as fp32 on the device: the tensor itself where it is that already."""
+    if t.dtype == torch.float32 and t.device == device:
+        return t
+    return t.reshape(-1)[:1].to(device=device, dtype=torch.float32).contiguous()
+
+
 def check(fn: str, code: int) -> None:
     if code != OK:
         if code == ERR_NOKERNEL:

@@ -115,11 +115,13 @@ def decode_params(impl, q, kv_c_and_k_pe_cache, attn_metadata, layer, out, lse):
     rope_w = impl.rms_offset - rank
     if isinstance(q, tuple):
         q_nope, q_pe = q
+        w_nope, w_pe = q_nope.shape[-1], q_pe.shape[-1]
     else:
-        q_nope, q_pe = q[..., :rank], q[..., rank:]
-    if q_nope.shape[-1] != rank or q_pe.shape[-1] < rope_w:
-        raise ValueError(f"query widths {q_nope.shape[-1]} / {q_pe.shape[-1]} do not cover rank {rank} "
-                         f"and the rope window {rope_w}")
+        # one tensor holds both: its own strides, the rope part `rank` columns in
+        q_nope = q_pe = q
+        w_nope, w_pe = min(q.shape[-1], rank), max(q.shape[-1] - rank, 0)
+    if w_nope != rank or w_pe < rope_w:
+        raise ValueError(f"query widths {w_nope} / {w_pe} do not cover rank {rank} and the rope window {rope_w}")
     if impl.mla_local_heads and q_nope.shape[1] != impl.mla_local_heads:
         raise ValueError(f"{q_nope.shape[1]} query heads, the cache rows hold rms for {impl.mla_local_heads}")
     # vLLM's MLA cache is [num_blocks, block_size, head_size]; the paged-row view adds the kv-head
@@ -138,6 +140,8 @@ def decode_params(impl, q, kv_c_and_k_pe_cache, attn_metadata, layer, out, lse):
                      out=out, lse=lse, d_c=rank, rope_w=rope_w, rms_offset=impl.rms_offset, rms_mode=rms_mode,
                      kv=kv, page_size=page_size, sm_scale=impl.scale, k_scale=k_scale,
                      qrows=1, groups=1, rms_heads=q_nope.shape[1], num_splits=0)
+    if q_pe is q_nope and rope_w > 0:
+        p.q_pe = q.data_ptr() + rank * q.element_size()
     if qrows > 1:
         p.qrows = fold_rows(p, qrows)
     return p
@@ -171,7 +175,7 @@ def forward_mqa(impl, q, kv_c_and_k_pe_cache, attn_metadata, layer):
         ws.reserve(need, q0.device)
     p.workspace = ws.buf.data_ptr()
     p.workspace_bytes = ws.buf.numel()
-    _lib.check("qmla_decode", _lib.lib().qmla_decode(p, torch.cuda.current_stream().cuda_stream))
+    _lib.check("qmla_decode", _lib.lib().qmla_decode(p, _lib.stream()))
     return out, lse
 
 

@@ -20,7 +20,7 @@ _RMS_WRITE = {"log8": _lib.RMS_LOG8, "bf16": _lib.RMS_BF16_BYTES, "e4m3": _lib.R
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return _lib.stream()
 
 
 def cache_write(kv_c: torch.Tensor, k_pe: torch.Tensor, kv_cache: torch.Tensor, slot_mapping: torch.Tensor, *,
@@ -34,9 +34,7 @@ def cache_write(kv_c: torch.Tensor, k_pe: torch.Tensor, kv_cache: torch.Tensor, 
     p, keep = cache_write_params(kv_c, k_pe, kv_cache, slot_mapping, d_c=d_c, rope_w=rope_w, rms_heads=rms_heads,
                                  kv_fp8=kv_fp8, rms=rms, k_scale=k_scale)
     _lib.check("qmla_cache_write", _lib.lib().qmla_cache_write(ctypes.byref(p), _stream()))
-    cur = torch.cuda.current_stream()
-    for t in keep:
-        t.record_stream(cur)
+    _lib.keep_alive(keep)
 
 
 def cache_write_params(kv_c: torch.Tensor, k_pe: torch.Tensor, kv_cache: torch.Tensor, slot_mapping: torch.Tensor,
@@ -44,7 +42,7 @@ def cache_write_params(kv_c: torch.Tensor, k_pe: torch.Tensor, kv_cache: torch.T
                        rms: str = "log8", k_scale: torch.Tensor | None = None):
     """The `qmla_cache_write_params` of a `cache_write` call, and the tensors it points into that the
     caller must keep alive (converted copies). For callers that launch the same write repeatedly."""
-    slots = slot_mapping.reshape(-1)
+    slots = slot_mapping if slot_mapping.dim() == 1 else slot_mapping.reshape(-1)
     n = slots.shape[0]
     if kv_fp8 is None:
         kv_fp8 = kv_cache.dtype in (torch.uint8, torch.float8_e4m3fn)
@@ -55,13 +53,13 @@ def cache_write_params(kv_c: torch.Tensor, k_pe: torch.Tensor, kv_cache: torch.T
             raise ValueError("cache_write: every tensor must live on the GPU")
     if kv_c.dtype != torch.bfloat16 or k_pe.dtype != torch.bfloat16:
         raise TypeError("cache_write: kv_c and k_pe must be bf16")
-    kv_c2 = kv_c.reshape(kv_c.shape[0], -1)
-    k_pe2 = k_pe.reshape(k_pe.shape[0], -1)
+    kv_c2, k_pe2 = _lib.rows2d(kv_c), _lib.rows2d(k_pe)
     if kv_c2.shape[0] < n or k_pe2.shape[0] < n:
         raise ValueError("cache_write: fewer input rows than slots")
     if kv_c2.stride(-1) != 1 or k_pe2.stride(-1) != 1:
         raise ValueError("cache_write: rows must be contiguous in their last dimension")
-    slots = slots.to(torch.int64)
+    if slots.dtype != torch.int64:
+        slots = slots.to(torch.int64)
     p = _lib.CacheWriteParams()
     p.kv_c, p.kv_c_stride = kv_c2.data_ptr(), kv_c2.stride(0)
     p.k_pe, p.k_pe_stride = k_pe2.data_ptr(), k_pe2.stride(0)
@@ -72,7 +70,7 @@ def cache_write_params(kv_c: torch.Tensor, k_pe: torch.Tensor, kv_cache: torch.T
         p.rms_mode = _lib.RMS_NONE if rms == "none" else _RMS_WRITE[rms]
         if k_scale is None:
             raise ValueError("cache_write: FP8 caches need k_scale")
-        ks = k_scale.reshape(-1)[:1].to(device=kv_cache.device, dtype=torch.float32).contiguous()
+        ks = _lib.as_scale(k_scale, kv_cache.device)
         p.k_scale = ks.data_ptr()
     else:
         p.kv_dtype = _lib.KV_BF16
@@ -121,9 +119,7 @@ def gather_cache(*, src_cache: torch.Tensor, dst: torch.Tensor, block_table: tor
                             token_to_seq=token_to_seq, num_tokens=num_tokens, kv_cache_dtype=kv_cache_dtype,
                             scale=scale, seq_starts=seq_starts, mla_rms=mla_rms)
     _lib.check("qmla_gather", _lib.lib().qmla_gather(ctypes.byref(p), _stream()))
-    cur = torch.cuda.current_stream()
-    for t in keep:
-        t.record_stream(cur)
+    _lib.keep_alive(keep)
 
 
 def gather_params(*, src_cache: torch.Tensor, dst: torch.Tensor, block_table: torch.Tensor,
@@ -141,10 +137,10 @@ def gather_params(*, src_cache: torch.Tensor, dst: torch.Tensor, block_table: to
             raise ValueError("gather_cache: every tensor must live on the GPU")
     if dst.dtype not in (torch.bfloat16, torch.float16):
         raise TypeError("gather_cache: dst must be bf16 or fp16")
-    dst2 = dst.reshape(dst.shape[0], -1)
+    dst2 = _lib.rows2d(dst)
     if dst2.stride(-1) != 1 or dst2.shape[0] < num_tokens:
         raise ValueError("gather_cache: dst rows must be contiguous and cover num_tokens")
-    i32 = lambda t: t.to(torch.int32).contiguous()
+    i32 = lambda t: t if t.dtype == torch.int32 and t.is_contiguous() else t.to(torch.int32).contiguous()
     bt, cu, t2s = i32(block_table), i32(cu_seq_lens), i32(token_to_seq)
     ss = i32(seq_starts) if seq_starts is not None else None
     p = _lib.GatherParams()
@@ -156,7 +152,7 @@ def gather_params(*, src_cache: torch.Tensor, dst: torch.Tensor, block_table: to
         off, nh = mla_rms[:2]
         mode = mla_rms[2] if len(mla_rms) > 2 else "bf16"
         p.kv_dtype, p.rms_mode, p.rms_offset, p.rms_heads = _lib.KV_FP8, _RMS_GATHER[mode], off, nh
-        sc = scale.reshape(-1)[:1].to(device=dst.device, dtype=torch.float32).contiguous()
+        sc = _lib.as_scale(scale, dst.device)
         p.scale = sc.data_ptr()
     else:
         p.kv_dtype, p.row_elems = _lib.KV_BF16, src_cache.reshape(src_cache.shape[0], src_cache.shape[1], -1).shape[-1]

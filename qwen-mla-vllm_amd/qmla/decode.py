@@ -69,7 +69,7 @@ def _rms_mode(kv: int, rms_offset: int, rms_bf16: bool, rms_log8: bool) -> int:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return _lib.stream()
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -277,26 +277,21 @@ def forward(q_nope, q_rope, kv_cache, block_table, seq_lens, *, d_c=None, rope_w
         k_scale = torch.tensor(float(k_scale), dtype=torch.float32, device=q_nope.device)
     if qrows > 1 and rows % qrows:
         raise ValueError(f"rows {rows} not a multiple of qrows {qrows}")
-    if qrows > 1:
-        probe = build_params(q_nope=q_nope, q_pe=q_rope, kv_cache=kv_cache, block_table=block_table,
-                             seq_lens=seq_lens, out=out, lse=lse, d_c=d_c, rope_w=rope_w, rms_offset=rms_offset,
-                             rms_mode=mode, kv=kv, page_size=page_size, sm_scale=sm_scale, logit_cap=logit_cap,
-                             groups=groups, rms_heads=rms_heads, num_splits=num_splits)
-        qrows = fold_rows(probe, qrows)
-    args = dict(q_nope=q_nope, q_pe=q_rope, kv_cache=kv_cache, block_table=block_table, seq_lens=seq_lens,
-                out=out, lse=lse, d_c=d_c, rope_w=rope_w, rms_offset=rms_offset, rms_mode=mode, kv=kv,
-                page_size=page_size, sm_scale=sm_scale, k_scale=k_scale, logit_cap=logit_cap, qrows=qrows,
-                groups=groups, rms_heads=rms_heads, num_splits=num_splits,
-                split_align=16 if page_size % 16 == 0 else 0, num_workgroups=num_workgroups, status=status)
+    p = build_params(q_nope=q_nope, q_pe=q_rope, kv_cache=kv_cache, block_table=block_table, seq_lens=seq_lens,
+                     out=out, lse=lse, d_c=d_c, rope_w=rope_w, rms_offset=rms_offset, rms_mode=mode, kv=kv,
+                     page_size=page_size, sm_scale=sm_scale, k_scale=k_scale, logit_cap=logit_cap, groups=groups,
+                     rms_heads=rms_heads, num_splits=num_splits, split_align=16 if page_size % 16 == 0 else 0,
+                     num_workgroups=num_workgroups, status=status)
+    if qrows != 1:
+        p.qrows = fold_rows(p, qrows) if qrows > 1 else qrows
     lib = _lib.lib()
     ws_t = None
-    ws_strides = (0, 0, 0)
     if num_splits > 1:
         ws_t = torch.empty(rows, H, num_splits, dv + 1, dtype=torch.float32, device=q_nope.device) \
             if workspace is None else workspace
-        ws_strides = (ws_t.stride(0), ws_t.stride(1), ws_t.stride(2))
+        p.ws_stride_row, p.ws_stride_head, p.ws_stride_split = ws_t.stride(0), ws_t.stride(1), ws_t.stride(2)
     elif num_splits == 0:
-        need = workspace_bytes(build_params(**args))
+        need = workspace_bytes(p)
         if isinstance(workspace, Workspace):
             ws_t = workspace.reserve(need, q_nope.device)
         elif workspace is not None:
@@ -304,6 +299,7 @@ def forward(q_nope, q_rope, kv_cache, block_table, seq_lens, *, d_c=None, rope_w
         else:
             w = _default_ws.setdefault(q_nope.device, Workspace())
             ws_t = w.reserve(need, q_nope.device)
-    p = build_params(workspace=ws_t, ws_strides=ws_strides, **args)
+    if ws_t is not None:
+        p.workspace, p.workspace_bytes = ws_t.data_ptr(), ws_t.numel() * ws_t.element_size()
     _lib.check("qmla_decode", lib.qmla_decode(p, _stream()))
     return out, lse

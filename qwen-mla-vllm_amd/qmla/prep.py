@@ -58,10 +58,8 @@ def mla_decode_prep(positions: torch.Tensor, q: torch.Tensor, latent: torch.Tens
                                        head_offset=head_offset, rope_group=rope_group, rope_first=rope_first,
                                        rope_span=rope_span, declared_rope=declared_rope, eps=eps, rope_sec=rope_sec,
                                        q_out=q_out, k_pe=k_pe)
-    _lib.check("qmla_prep", _lib.lib().qmla_prep(ctypes.byref(p), torch.cuda.current_stream().cuda_stream))
-    s = torch.cuda.current_stream()
-    for t in keep:
-        t.record_stream(s)
+    _lib.check("qmla_prep", _lib.lib().qmla_prep(ctypes.byref(p), _lib.stream()))
+    _lib.keep_alive(keep)
     return q_out, k_pe
 
 
@@ -87,8 +85,8 @@ def prep_params(positions, q, latent, k_rope, k_up_raw, k_gain, cos_sin_cache, *
         raise TypeError("mla_decode_prep: cos_sin_cache must be a contiguous [max_pos, rd] bf16/fp32/fp16 table")
     if q.stride(-1) != 1:
         raise ValueError("mla_decode_prep: q's last dimension must be contiguous")
-    lat = latent.reshape(-1, d_c)
-    kr = k_rope.reshape(k_rope.shape[0], -1)
+    lat = latent if latent.dim() == 2 and latent.numel() > 0 else latent.reshape(-1, d_c)
+    kr = _lib.rows2d(k_rope)
     if lat.shape[0] < n or kr.shape[0] < n or lat.stride(-1) != 1 or kr.stride(-1) != 1:
         raise ValueError("mla_decode_prep: latent / k_rope need n contiguous rows")
     if kr.shape[1] % rd:
@@ -97,10 +95,10 @@ def prep_params(positions, q, latent, k_rope, k_up_raw, k_gain, cos_sin_cache, *
     ku = k_up_raw.contiguous()
     if tuple(ku.shape) != (H * nope, d_c):
         raise ValueError(f"mla_decode_prep: k_up_raw must be [{H * nope}, {d_c}], got {tuple(ku.shape)}")
-    gain = k_gain.to(torch.float32).contiguous()
+    gain = (k_gain if k_gain.dtype == torch.float32 else k_gain.to(torch.float32)).contiguous()
     if gain.numel() < rd:
         raise ValueError("mla_decode_prep: k_gain needs rope_dim entries")
-    pos = positions.to(torch.int64)
+    pos = positions if positions.dtype == torch.int64 else positions.to(torch.int64)
     if pos.dim() == 1:
         pos = pos.contiguous()
         rows, prs, sec = 1, 0, None
@@ -122,7 +120,7 @@ def prep_params(positions, q, latent, k_rope, k_up_raw, k_gain, cos_sin_cache, *
         k_pe = torch.empty(n, declared_rope, dtype=torch.bfloat16, device=dev)
     if q_out.dtype != torch.bfloat16 or k_pe.dtype != torch.bfloat16 or q_out.stride(-1) != 1 or k_pe.stride(-1) != 1:
         raise ValueError("mla_decode_prep: outputs must be bf16 with a contiguous last dimension")
-    kp = k_pe.reshape(k_pe.shape[0], -1)
+    kp = _lib.rows2d(k_pe)
 
     p = _lib.PrepParams()
     p.q, p.q_token_stride, p.q_head_stride = q.data_ptr(), q.stride(0), q.stride(1)
