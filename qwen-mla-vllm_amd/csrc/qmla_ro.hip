@@ -252,11 +252,20 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
     return d;
   };
 
-  // window planning cursor (wave 0 only)
+  // window planning cursor (first DMA wave only)
   int cb = fixed ? (int)blockIdx.y : b0, ctok = 0, cp = c0;
+  // the range's first piece, if it has one, is the cursor's request: its query is loaded and converted
+  // while a DMA wave plans the window and the first tile is in flight, not in the first step
+  bool q_ready = false;
+  if constexpr (ROLE == COMPUTE) {
+    if (live) load_q(cb);
+    q_ready = true;
+  }
 
   for (;;) {
-    if (w == 0) plan_window<kPlanSwitchRo>(p, sm, fixed, lo, hi, cb, ctok, cp);
+    if constexpr (ROLE == DMA) {
+      if (dw == 0) plan_window<kPlanSwitchRo>(p, sm, fixed, lo, hi, cb, ctok, cp);
+    }
     __syncthreads();
     const int nseg = sm.win[0], ntot = sm.win[1], npg = sm.win[2], more = sm.win[3];
     if (nseg == 0) break;
@@ -410,7 +419,8 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
             lpart = 0.f;
 #pragma unroll
             for (int c = 0; c < C::CB; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (live) load_q(d.req);
+            if (live && !q_ready) load_q(d.req);
+            q_ready = false;
           }
           const int lr = d.L - (qrows - 1 - jq);
           lim = rok ? (lr < d.te ? lr : d.te) : 0;
@@ -565,7 +575,7 @@ __global__ __launch_bounds__(C::NTHR, 1) void ro_kernel(const KParams p) {
   const int wr = blockIdx.x;
   int lo = 0, hi = 0, b0 = 0, c0 = 0;
   if (!fixed) {
-    if (wr == 0 && wv == 1) store_plan<kPlanSwitchRo>(p);   // for the balanced combine
+    if (wr == 0 && wv == C::NCW + 1) store_plan<kPlanSwitchRo>(p);   // for the balanced combine
     const BalRange r = balanced_range<kPlanSwitchRo>(p, wr);
     lo = r.lo;
     hi = r.hi;

@@ -381,11 +381,21 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
     zero_acc();
   };
 
-  // window planning cursor (wave 0 only): request, token, plan prefix of the request
+  // window planning cursor (first value wave only): request, token, plan prefix of the request
   int cb = fixed ? (int)blockIdx.y : b0, ctok = 0, cp = c0;
+  // the range's first piece, if it has one, is the cursor's request: its query is loaded and converted
+  // while a value wave plans the window and the first tile is in flight, not in the first step
+  bool q_ready = false;
+  if constexpr (QS && C::G == 1) {
+    load_q(cb, 0);
+    set_q(0);
+    q_ready = true;
+  }
 
   for (;;) {
-    if (w == 0) plan_window<kPlanSwitchWs>(p, sm, fixed, lo, hi, cb, ctok, cp);
+    if constexpr (ROLE == VALUE) {
+      if (vw == 0) plan_window<kPlanSwitchWs>(p, sm, fixed, lo, hi, cb, ctok, cp);
+    }
     __syncthreads();
     const int nseg = sm.win[0], ntot = sm.win[1], npg = sm.win[2], more = sm.win[3];
     if (nseg == 0) break;
@@ -500,7 +510,7 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
             s_fl = d.fl;
             if (d.fl & SEG_FIRST) {
               if constexpr (C::G == 1) {
-                load_q(d.req, 0);   // in flight during the reads below, converted after them
+                if (!q_ready) load_q(d.req, 0);   // in flight during the reads below, converted after them
               } else {
                 // three row blocks: the query switches here, before this tile's reads (the previous
                 // request's softmax state does not depend on the query or its scale)
@@ -588,7 +598,10 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
                 mref[m] = kNegInf;
                 lpart[m] = 0.f;
               }
-              if constexpr (C::G == 1) set_q(0);
+              if constexpr (C::G == 1) {
+                if (!q_ready) set_q(0);
+                q_ready = false;
+              }
             }
           }
           // ---- S^T = K . Q^T as the K rows arrive ----
@@ -895,7 +908,7 @@ __global__ __launch_bounds__(C::NTHR, 1) void ws_kernel(const KParams p) {
   }
   int lo = 0, hi = 0, b0 = 0, c0 = 0;
   if (!fixed) {
-    if (wr == 0 && hz == 0 && wv == 1) store_plan<kPlanSwitchWs>(p);   // for the balanced combine
+    if (wr == 0 && hz == 0 && wv == 5) store_plan<kPlanSwitchWs>(p);   // for the balanced combine
     const BalRange r = balanced_range<kPlanSwitchWs>(p, wr);
     lo = r.lo;
     hi = r.hi;

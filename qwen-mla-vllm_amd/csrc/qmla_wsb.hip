@@ -339,11 +339,20 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
     zero_acc();
   };
 
-  // window planning cursor (wave 0 only): request, token, plan prefix of the request
+  // window planning cursor (first value wave only): request, token, plan prefix of the request
   int cb = fixed ? (int)blockIdx.y : b0, ctok = 0, cp = c0;
+  // the range's first piece, if it has one, is the cursor's request: its query is loaded and converted
+  // while a value wave plans the window and the first tile is in flight, not in the first step
+  bool q_ready = false;
+  if constexpr (QS) {
+    load_q(cb);
+    q_ready = true;
+  }
 
   for (;;) {
-    if (w == 0) plan_window<kPlanSwitchWs, PIDB>(p, sm, fixed, lo, hi, cb, ctok, cp);
+    if constexpr (!QS) {
+      if (w == 0) plan_window<kPlanSwitchWs, PIDB>(p, sm, fixed, lo, hi, cb, ctok, cp);
+    }
     __syncthreads();
     const int nseg = sm.win[0], ntot = sm.win[1], npg = sm.win[2], more = sm.win[3];
     if (nseg == 0) break;
@@ -453,7 +462,8 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
             s_nt = d.nt;
             s_fl = d.fl;
             if (d.fl & SEG_FIRST) {
-              load_q(d.req);
+              if (!q_ready) load_q(d.req);
+              q_ready = false;
               mref = kNegInf;
               lpart = 0.f;
             }
