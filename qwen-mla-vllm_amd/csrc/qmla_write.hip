@@ -11,12 +11,42 @@
 #include <stdint.h>
 
 #include "qmla.h"
+#include "qmla_common.h"
 #include "qmla_device.h"
 
 namespace qmla {
-// rows from which the writer and the gather take several rows a wave (measured on MI355X: at 16384
-// rows one row a wave is as fast or faster, at 262144 several rows a wave 23% / 37% faster)
-constexpr int kMultiRowMin = 65536;
+// token / page_size for tokens below 2^31 by multiplication (page_magic); mul 0: a 64-bit division
+// (cache of 2^31 slots or more)
+struct PageDiv {
+  uint32_t mul;
+  int sh, size;
+};
+static PageDiv page_div_of(int page_size, int64_t tokens) {
+  PageDiv d{0u, 0, page_size};
+  if (tokens <= 0x7fffffff) page_magic(page_size, d.mul, d.sh);
+  return d;
+}
+__device__ __forceinline__ int64_t page_of(const PageDiv& d, int64_t tok) {
+  return d.mul ? (int64_t)(((uint64_t)(uint32_t)tok * d.mul) >> d.sh) : tok / d.size;
+}
+// flat slots of a wave's rows: slot q of rows of n slots is slot (q - r n) of row r = q / n, from a
+// 24-bit multiplication (q < 2^10, exact below 2^20 / n)
+__device__ __forceinline__ uint32_t flat_mul(int n) { return ((1u << 20) + (uint32_t)n - 1) / (uint32_t)n; }
+__device__ __forceinline__ int flat_row(int q, uint32_t mul) { return (int)(__umul24((uint32_t)q, mul) >> 20); }
+__device__ __forceinline__ int64_t lane64(int64_t v, int lane) {   // another lane's value
+  const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)v, lane), hi = (uint32_t)__shfl((int)(uint32_t)((uint64_t)v >> 32), lane);
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ int64_t uniform64(int64_t v, int lane) {   // lane's value as a scalar
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)v >> 32), lane);
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+// rows from which FP8 rows are written and gathered several to a wave. Writer: 1000 rows of rank 512
+// 3.2 us at one a wave, 3.3 at two; 4000 rows 4.5 and 3.9. Gather: 1000 rows 3.6 and 3.8, 12001 rows
+// 10.7 and 7.7 (rank 768: 12.1 and 9.8, rank 1792 16.9 and 15.1). Four rows a wave for rows below 1024
+// bytes: 20000 rows 10.9 and 10.5, 200000 rows 100 and 79 (rank 768: 131 and 128)
+constexpr int kWriteRowsMin = 2048, kGatherRowsMin = 4096, kGatherRows4Min = 16384;
 namespace wr {
 
 constexpr int ROWS_PER_WG = 4;
@@ -31,7 +61,7 @@ struct WParams {
   const float* k_scale;
   char* cache;
   int64_t page_stride, token_stride;
-  int page_size;
+  PageDiv page;
   int64_t num_slots;
 };
 
@@ -84,14 +114,15 @@ __device__ __forceinline__ uint32_t log8_code_fast(float r) {
   return (uint32_t)(c < 0.0f ? 0.0f : (c > 255.0f ? 255.0f : c));
 }
 
+// One wave a row: bf16 caches, and FP8 rows outside write_rows_kernel's limits.
 __global__ __launch_bounds__(64 * ROWS_PER_WG) void write_kernel(const WParams p) {
   const int lane = threadIdx.x & 63;
-  const int row = (int)blockIdx.x * ROWS_PER_WG + (int)(threadIdx.x >> 6);
+  const int row = (int)blockIdx.x * ROWS_PER_WG + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   if (row >= p.n) return;
   int64_t slot = p.slots[row];
   if (slot < 0) slot = 0;
   if (slot >= p.num_slots) return;
-  const int64_t page = slot / p.page_size, tok = slot - page * p.page_size;
+  const int64_t page = page_of(p.page, slot), tok = slot - page * p.page.size;
   char* dst = p.cache + page * p.page_stride + tok * p.token_stride;
   const uint16_t* kc = p.kv_c + (int64_t)row * p.kv_c_stride;
   const uint16_t* kp = p.k_pe + (int64_t)row * p.k_pe_stride;
@@ -113,7 +144,7 @@ __global__ __launch_bounds__(64 * ROWS_PER_WG) void write_kernel(const WParams p
     for (int h = lane; h < p.rms_heads; h += 64) {
       const uint16_t rb = kp[p.rope_w + h];
       if (p.rms_mode == QMLA_RMS_LOG8) {
-        rt[h] = (char)log8_code(bf16_to_f32(rb));
+        rt[h] = (char)log8_code_fast(bf16_to_f32(rb));
       } else if (p.rms_mode == QMLA_RMS_BF16_BYTES) {
         rt[2 * h] = (char)(rb & 0xFF);
         rt[2 * h + 1] = (char)(rb >> 8);
@@ -130,62 +161,100 @@ __global__ __launch_bounds__(64 * ROWS_PER_WG) void write_kernel(const WParams p
   }
 }
 
-// FP8 rows with latents up to 512 * NCL columns, a rope up to 512 and up to 64 rms heads: one wave
-// writes WROWS rows, all of their input loads in flight before the first conversion (a lone row's
-// load latency would otherwise bound a wave), the same bytes as write_kernel.
-constexpr int WROWS = 4;
-template <int NCL>
-__global__ __launch_bounds__(256) void write_fp8_kernel(const WParams p) {
+// FP8 rows: one wave writes R rows. Whole 512-column blocks of a row go one 8-column chunk to a lane
+// (row addresses in scalar registers); the chunks left over, the 1-7 rope elements before an rms tail
+// that is not 8-aligned, and the rms elements of the R rows are each dealt out flat over the wave.
+// Every load is in flight before the first conversion. The same bytes as write_kernel.
+//
+// What bounds it: below some 20000 rows the launch of the waves and each one's chain of slot, row and
+// store, above that memory (60000 rows of rank 512: 108 MB in 21 us, 5.1 TB/s). 12001 rows of rank
+// 512 / 768 / 1792 at one row a wave 9.1 / 11.0 / 15.8 us (write_kernel), two rows 6.7 / 8.4 / 14.7,
+// four 6.6 / 9.0 / 16.7, eight 7.8 / 11.5 / 19.9; 200000 rows of rank 512 and 768, two rows 71 / 116,
+// four rows with every row's rope and tail passes of its own 75 / 115 (the form before this one).
+template <int R, int NF>
+__global__ __launch_bounds__(256) void write_rows_kernel(const WParams p) {
   const int lane = threadIdx.x & 63;
-  const int r0 = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * WROWS;
+  const int r0 = ((int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * R;
   if (r0 >= p.n) return;
+  const int nr = p.n - r0 < R ? p.n - r0 : R;
+  const int nfull = p.d_c >> 9, rem = (p.d_c >> 3) & 63, nrp = p.rope_w >> 3, npre = p.rope_w & 7;
+  const int ns = rem + nrp, heads = p.rms_mode == QMLA_RMS_NONE ? 0 : p.rms_heads;
+  const uint32_t ms = ns > 0 ? flat_mul(ns) : 0u, mh = heads > 0 ? flat_mul(heads) : 0u;
+  const uint16_t* kc = p.kv_c + (int64_t)r0 * p.kv_c_stride;
+  const uint16_t* kp = p.k_pe + (int64_t)r0 * p.k_pe_stride;
+  // ---- loads (rows past the end repeat the last row's) ----
+  const int64_t slot0 = p.slots[r0 + (lane < nr ? lane : nr - 1)];
   const float inv = 1.0f / *p.k_scale;
-  const int r8 = p.rope_w & ~7;
-  uint4 lat[WROWS][NCL], rp[WROWS];
-  uint16_t rt[WROWS], rm[WROWS];
-  int64_t slot[WROWS];
+  uint4 lat[R][NF], fl[R];
+  uint16_t rm[R], pre = 0;
 #pragma unroll
-  for (int i = 0; i < WROWS; ++i) {
-    const int row = r0 + i < p.n ? r0 + i : p.n - 1;   // past the end: a valid row, not written
-    const uint16_t* kc = p.kv_c + (int64_t)row * p.kv_c_stride;
-    const uint16_t* kp = p.k_pe + (int64_t)row * p.k_pe_stride;
-    slot[i] = p.slots[row];
+  for (int i = 0; i < R; ++i) {
+    const uint16_t* row = kc + (int64_t)(i < nr ? i : nr - 1) * p.kv_c_stride;
 #pragma unroll
-    for (int k = 0; k < NCL; ++k) {
-      const int c = 8 * lane + 512 * k;
-      lat[i][k] = c < p.d_c ? *reinterpret_cast<const uint4*>(kc + c) : make_uint4(0u, 0u, 0u, 0u);
-    }
-    rp[i] = 8 * lane < r8 ? *reinterpret_cast<const uint4*>(kp + 8 * lane) : make_uint4(0u, 0u, 0u, 0u);
-    rt[i] = lane < p.rope_w - r8 ? kp[r8 + lane] : (uint16_t)0;
-    rm[i] = lane < p.rms_heads ? kp[p.rope_w + lane] : (uint16_t)0;
+    for (int k = 0; k < NF; ++k)
+      if (k < nfull) lat[i][k] = *reinterpret_cast<const uint4*>(row + 8 * (lane + 64 * k));
   }
 #pragma unroll
-  for (int i = 0; i < WROWS; ++i) {
-    if (r0 + i >= p.n) break;
-    int64_t sl = slot[i];
-    if (sl < 0) sl = 0;
-    if (sl >= p.num_slots) continue;
-    const int64_t page = sl / p.page_size, tok = sl - page * p.page_size;
-    char* dst = p.cache + page * p.page_stride + tok * p.token_stride;
-#pragma unroll
-    for (int k = 0; k < NCL; ++k) {
-      const int c = 8 * lane + 512 * k;
-      if (c < p.d_c) *reinterpret_cast<uint2*>(dst + c) = quant8r(lat[i][k], inv);
+  for (int i = 0; i < R; ++i) {
+    const int q = lane + 64 * i;
+    if (64 * i < R * ns && q < nr * ns) {
+      const int r = flat_row(q, ms), c = q - r * ns;
+      fl[i] = *reinterpret_cast<const uint4*>(c < rem ? kc + r * p.kv_c_stride + 512 * nfull + 8 * c
+                                                     : kp + r * p.k_pe_stride + 8 * (c - rem));
     }
-    if (8 * lane < r8) *reinterpret_cast<uint2*>(dst + p.d_c + 8 * lane) = quant8r(rp[i], inv);
-    if (lane < p.rope_w - r8)
-      dst[p.d_c + r8 + lane] = (char)(pack_e4m3(sat448(bf16_to_f32(rt[i]), inv), 0.f, 0.f, 0.f) & 0xFF);
-    if (lane < p.rms_heads) {
-      char* rtl = dst + p.d_c + p.rope_w;
-      if (p.rms_mode == QMLA_RMS_LOG8) {
-        rtl[lane] = (char)log8_code_fast(bf16_to_f32(rm[i]));
-      } else if (p.rms_mode == QMLA_RMS_BF16_BYTES) {
-        rtl[2 * lane] = (char)(rm[i] & 0xFF);
-        rtl[2 * lane + 1] = (char)(rm[i] >> 8);
-      } else if (p.rms_mode == QMLA_RMS_E4M3) {
-        rtl[lane] = (char)(pack_e4m3(sat448(bf16_to_f32(rm[i]), inv), 0.f, 0.f, 0.f) & 0xFF);
+    if (64 * i < R * heads && q < nr * heads) {
+      const int r = flat_row(q, mh);
+      rm[i] = kp[r * p.k_pe_stride + p.rope_w + q - r * heads];
+    }
+  }
+  const int pr = npre > 0 ? lane / npre : R, pe = lane - pr * npre;   // this lane's pre-tail element
+  if (pr < nr) pre = kp[pr * p.k_pe_stride + 8 * nrp + pe];
+  // ---- lane r: byte offset of row r0 + r's slot, or -1 (nothing to write) ----
+  const int64_t slot = slot0 < 0 ? 0 : slot0;
+  int64_t off = -1;
+  if (lane < nr && slot < p.num_slots) {
+    const int64_t page = page_of(p.page, slot);
+    off = page * p.page_stride + (slot - page * p.page.size) * p.token_stride;
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int64_t o = uniform64(off, i);
+    if (o < 0) continue;
+#pragma unroll
+    for (int k = 0; k < NF; ++k)
+      if (k < nfull) *reinterpret_cast<uint2*>(p.cache + o + 8 * (lane + 64 * k)) = quant8r(lat[i][k], inv);
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int q = lane + 64 * i;
+    if (64 * i < R * ns) {   // wave-uniform
+      const int r = q < nr * ns ? flat_row(q, ms) : 0;
+      const int64_t o = lane64(off, r);
+      const int c = q - r * ns;
+      if (q < nr * ns && o >= 0)
+        *reinterpret_cast<uint2*>(p.cache + o + 8 * (c < rem ? 64 * nfull + c : (p.d_c >> 3) + c - rem)) = quant8r(fl[i], inv);
+    }
+    if (64 * i < R * heads) {
+      const int r = q < nr * heads ? flat_row(q, mh) : 0;
+      const int64_t o = lane64(off, r);
+      const int h = q - r * heads;
+      if (q < nr * heads && o >= 0) {
+        char* rt = p.cache + o + p.d_c + p.rope_w;
+        if (p.rms_mode == QMLA_RMS_LOG8) {
+          rt[h] = (char)log8_code_fast(bf16_to_f32(rm[i]));
+        } else if (p.rms_mode == QMLA_RMS_BF16_BYTES) {
+          rt[2 * h] = (char)(rm[i] & 0xFF);
+          rt[2 * h + 1] = (char)(rm[i] >> 8);
+        } else {
+          rt[h] = (char)(pack_e4m3(sat448(bf16_to_f32(rm[i]), inv), 0.f, 0.f, 0.f) & 0xFF);
+        }
       }
     }
+  }
+  if (npre > 0) {
+    const int64_t o = lane64(off, pr < nr ? pr : 0);
+    if (pr < nr && o >= 0)
+      p.cache[o + p.d_c + 8 * nrp + pe] = (char)(pack_e4m3(sat448(bf16_to_f32(pre), inv), 0.f, 0.f, 0.f) & 0xFF);
   }
 }
 
@@ -235,14 +304,13 @@ extern "C" int qmla_cache_write(const qmla_cache_write_params* p, void* stream) 
   k.cache = static_cast<char*>(p->cache);
   k.page_stride = p->page_stride;
   k.token_stride = p->token_stride;
-  k.page_size = p->page_size;
+  k.page = page_div_of(p->page_size, p->num_slots);
   k.num_slots = p->num_slots;
   void* args[] = {&k};
-  // large batches (a long prefill): WROWS rows a wave; smaller ones keep one row a wave, which
-  // spreads them over more waves
-  if (fp8 && p->n >= kMultiRowMin && p->d_c <= 1024 && p->rope_w <= 512 && p->rms_heads <= 64) {
-    const unsigned grid = (unsigned)((p->n + 4 * wr::WROWS - 1) / (4 * wr::WROWS));
-    const void* fn = p->d_c <= 512 ? (const void*)wr::write_fp8_kernel<1> : (const void*)wr::write_fp8_kernel<2>;
+  if (fp8 && p->n >= kWriteRowsMin && p->d_c <= 2047 && (p->d_c / 8) % 64 + p->rope_w / 8 <= 64 && p->rms_heads <= 64) {
+    constexpr int R = 2;
+    const unsigned grid = (unsigned)((p->n + 4 * R - 1) / (4 * R));
+    const void* fn = p->d_c < 1024 ? (const void*)wr::write_rows_kernel<R, 1> : (const void*)wr::write_rows_kernel<R, 3>;
     const hipError_t e = hipLaunchKernel(fn, dim3(grid), dim3(256), args, 0, (hipStream_t)stream);
     return e == hipSuccess ? QMLA_OK : QMLA_ERR_LAUNCH;
   }
@@ -263,7 +331,8 @@ constexpr int ROWS_PER_WG = 4;
 struct GParams {
   const char* cache;
   int64_t page_stride, token_stride;
-  int page_size, num_pages, kv_dtype, rms_mode, rms_offset, rms_heads, row_elems;
+  PageDiv page;
+  int num_pages, kv_dtype, rms_mode, rms_offset, rms_heads, row_elems;
   const float* scale;
   const int32_t* block_table;
   int64_t bt_stride;
@@ -298,20 +367,48 @@ __device__ __forceinline__ uint16_t to_out(float x, int dt) {
   return (uint16_t)(__builtin_bit_cast(uint16_t, (__bf16)x) | sign);
 }
 
-__global__ __launch_bounds__(64 * ROWS_PER_WG) void gather_kernel(const GParams p) {
-  const int lane = threadIdx.x & 63;
-  const int j = (int)blockIdx.x * ROWS_PER_WG + (int)(threadIdx.x >> 6);
-  if (j >= p.num_tokens) return;
+// log8 code -> 2^(-3 + code * 6/255), rounded once from double
+struct Log8Table {
+  float v[256];
+};
+constexpr Log8Table make_log8() {
+  Log8Table t{};
+  for (int c = 0; c < 256; ++c) {
+    const double x = -3.0 + c * (6.0 / 255.0);
+    const int n = (int)(x + 8.0) - 8;                          // floor
+    const double f = (x - n) * 0.693147180559945309417232121458;
+    double term = 1.0, sum = 1.0;                              // e^f, 0 <= f < ln 2
+    for (int k = 1; k < 28; ++k) {
+      term *= f / k;
+      sum += term;
+    }
+    t.v[c] = (float)(n >= 0 ? sum * (double)(1 << n) : sum / (double)(1 << -n));
+  }
+  return t;
+}
+__constant__ Log8Table kLog8 = make_log8();
+
+// byte offset in the cache of destination row j, or -1 (nothing to write)
+__device__ __forceinline__ int64_t row_offset(const GParams& p, int j) {
   const int s = p.token_to_seq[j];
-  if (s < 0 || s >= p.num_seqs) return;
+  if (s < 0 || s >= p.num_seqs) return -1;
   int64_t tok = (int64_t)j - p.cu_seq_lens[s];
   if (p.seq_starts) tok += p.seq_starts[s];
-  if (tok < 0) return;
-  const int64_t pi = tok / p.page_size;
-  if (pi >= p.bt_cols) return;
+  if (tok < 0 || tok >= (int64_t)p.bt_cols * p.page.size) return -1;
+  const int64_t pi = page_of(p.page, tok);
   const int blk = p.block_table[(int64_t)s * p.bt_stride + pi];
-  if (blk < 0 || blk >= p.num_pages) return;
-  const char* row = p.cache + (int64_t)blk * p.page_stride + (tok - pi * p.page_size) * p.token_stride;
+  if (blk < 0 || blk >= p.num_pages) return -1;
+  return (int64_t)blk * p.page_stride + (tok - pi * p.page.size) * p.token_stride;
+}
+
+// One wave a row: bf16 caches, and FP8 rows outside gather_rows_kernel's limits.
+__global__ __launch_bounds__(64 * ROWS_PER_WG) void gather_kernel(const GParams p) {
+  const int lane = threadIdx.x & 63;
+  const int j = (int)blockIdx.x * ROWS_PER_WG + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (j >= p.num_tokens) return;
+  const int64_t off = row_offset(p, j);
+  if (off < 0) return;
+  const char* row = p.cache + off;
   uint16_t* out = reinterpret_cast<uint16_t*>(p.dst) + (int64_t)j * p.dst_stride;
 
   if (p.kv_dtype == QMLA_KV_BF16) {
@@ -354,7 +451,7 @@ __global__ __launch_bounds__(64 * ROWS_PER_WG) void gather_kernel(const GParams 
   for (int h = lane; h < p.rms_heads; h += 64) {
     float v;
     if (p.rms_mode == QMLA_RMS_LOG8) {
-      v = (float)exp2(-3.0 + (double)tail[h] * (6.0 / 255.0));   // 2^(-3 + code*6/255)
+      v = kLog8.v[tail[h]];
     } else if (p.rms_mode == QMLA_RMS_BF16_BYTES) {
       const uint32_t bits = (uint32_t)tail[2 * h] | ((uint32_t)tail[2 * h + 1] << 8);
       if (p.dst_dtype == QMLA_DT_BF16) {
@@ -369,138 +466,110 @@ __global__ __launch_bounds__(64 * ROWS_PER_WG) void gather_kernel(const GParams 
   }
 }
 
-// FP8 rows whose latent + rope span at most 1024 bytes and whose rms tail holds at most 64 heads:
-// one wave gathers GROWS destination rows. Lanes 0 .. GROWS-1 resolve the rows' sequence, token and
-// page together (the per-row kernel waits for that chain of dependent loads once per row). The
-// rows' 8-byte chunks are then dealt out flat, chunk q of the wave to lane q % 64, so every issued
-// conversion is a full one (a row of 72 chunks would leave 56 lanes idle in its second pass), and
-// all their loads are in flight before the first conversion; likewise the rms elements. The same
-// values as gather_kernel.
-constexpr int GROWS = 8;
+// 8 e4m3 bytes -> scaled, in the destination dtype
 template <int DT>
-__global__ __launch_bounds__(256) void gather_fp8_kernel(const GParams p) {
-  constexpr int NQ = GROWS * 128 / 64;   // chunk passes at most (1024-byte rows)
-  constexpr int NT = GROWS * 64 / 64;    // rms passes at most (64 heads)
+__device__ __forceinline__ uint4 dequant8(const uint2 raw, float sc) {
+  const uint32_t w[2] = {raw.x, raw.y};
+  uint32_t o[4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int wv = (int)w[h];
+    const float f0 = e4m3_f32(wv, 0) * sc, f1 = e4m3_f32(wv, 1) * sc;
+    const float f2 = e4m3_f32(wv, 2) * sc, f3 = e4m3_f32(wv, 3) * sc;
+    o[2 * h] = (uint32_t)to_out(f0, DT) | ((uint32_t)to_out(f1, DT) << 16);
+    o[2 * h + 1] = (uint32_t)to_out(f2, DT) | ((uint32_t)to_out(f3, DT) << 16);
+  }
+  return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+// FP8 rows: one wave gathers R destination rows. Lanes 0 .. R-1 resolve the rows' sequence, token and
+// page together. Whole 512-byte blocks of a row go one 8-byte chunk to a lane (row addresses in scalar
+// registers); the chunks left over, the 1-7 bytes before an rms tail that is not 8-aligned, and the
+// rms elements of the R rows are each dealt out flat over the wave. Every load is in flight before the
+// first conversion. The same values as gather_kernel.
+//
+// What bounds it: as write_rows_kernel, the waves and their chain (sequence, page, row) below some 20000
+// rows, memory above. 20000 rows of rank 512 / 768 / 1792: 16.1 / 17.4 / 24.6 us at one row a wave with
+// a 64-bit division and an exp2 in double for each, 10.9 / 14.2 / 21.7 at two rows, 10.5 / 14.7 / 22.8
+// at four; 60000 rows 39 / 41 / 82 at one, 24.4 / 32.0 / 76 at two, 22.7 / 32.6 / 86 at four.
+template <int DT, int R, int NF>
+__global__ __launch_bounds__(256) void gather_rows_kernel(const GParams p) {
   const int lane = threadIdx.x & 63;
-  const int j0 = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * GROWS;
-  // the 256 log8 divisors, 2^(-3 + code*6/255) rounded once from double, one per thread (every
-  // thread of the workgroup takes part, before any leaves)
-  __shared__ float l8[256];
-  if (p.rms_mode == QMLA_RMS_LOG8) {
-    l8[threadIdx.x] = (float)exp2(-3.0 + (double)threadIdx.x * (6.0 / 255.0));
-    __syncthreads();
-  }
+  const int j0 = ((int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * R;
   if (j0 >= p.num_tokens) return;
-  // lane r < GROWS: byte offset of row j0 + r in the cache, or -1 (nothing to write)
-  int64_t roff = -1;
-  if (lane < GROWS && j0 + lane < p.num_tokens) {
-    const int j = j0 + lane;
-    const int s = p.token_to_seq[j];
-    if (s >= 0 && s < p.num_seqs) {
-      int64_t tok = (int64_t)j - p.cu_seq_lens[s];
-      if (p.seq_starts) tok += p.seq_starts[s];
-      if (tok >= 0) {
-        const int64_t pi = tok / p.page_size;
-        if (pi < p.bt_cols) {
-          const int blk = p.block_table[(int64_t)s * p.bt_stride + pi];
-          if (blk >= 0 && blk < p.num_pages)
-            roff = (int64_t)blk * p.page_stride + (tok - pi * p.page_size) * p.token_stride;
-        }
-      }
-    }
-  }
-  const int roff_lo = (int)(uint32_t)roff, roff_hi = (int)(uint32_t)((uint64_t)roff >> 32);
-  const int c8 = p.rms_offset & ~7, nch = c8 >> 3, npre = p.rms_offset - c8;
-  const int rb = p.rms_mode == QMLA_RMS_BF16_BYTES ? 2 : 1;
-  const int nel = nch + (npre > 0 ? 1 : 0);            // chunk slots a row: whole chunks + the pre-tail
-  const int total = GROWS * nel, nt = GROWS * p.rms_heads;
-  // q / nel and t / rms_heads from 24-bit multiplies (q, t < 2^11; exact below 2^20 / divisor)
-  const uint32_t mq = ((1u << 20) + nel - 1) / nel, mt = p.rms_heads > 0 ? ((1u << 20) + p.rms_heads - 1) / p.rms_heads : 0u;
-  uint2 raw[NQ];
-  uint32_t tb[NT];
-  uint32_t live = 0u;   // bit i: this lane's chunk slot of pass i belongs to a row to write
-#pragma unroll
-  for (int i = 0; i < NQ; ++i) {
-    raw[i] = make_uint2(0u, 0u);
-    if (64 * i < total) {   // wave-uniform
-      const int q = lane + 64 * i;
-      const int r = (int)(__umul24((uint32_t)(q < total ? q : 0), mq) >> 20);
-      const uint32_t lo = (uint32_t)__shfl(roff_lo, r), hi = (uint32_t)__shfl(roff_hi, r);
-      const int64_t ro = (int64_t)(((uint64_t)hi << 32) | lo);
-      if (q < total && ro >= 0) {
-        live |= 1u << i;
-        const int c = q - (int)__umul24((uint32_t)r, (uint32_t)nel);
-        if (c < nch) raw[i] = *reinterpret_cast<const uint2*>(p.cache + ro + 8 * c);
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < NT; ++i) {
-    tb[i] = 0u;
-    if (64 * i < nt) {
-      const int t = lane + 64 * i;
-      const int r = (int)(__umul24((uint32_t)(t < nt ? t : 0), mt) >> 20);
-      const uint32_t lo = (uint32_t)__shfl(roff_lo, r), hi = (uint32_t)__shfl(roff_hi, r);
-      const int64_t ro = (int64_t)(((uint64_t)hi << 32) | lo);
-      if (t < nt && ro >= 0) {
-        const int h = t - (int)__umul24((uint32_t)r, (uint32_t)p.rms_heads);
-        const unsigned char* tail = reinterpret_cast<const unsigned char*>(p.cache + ro) + p.rms_offset;
-        tb[i] = rb == 2 ? ((uint32_t)tail[2 * h] | ((uint32_t)tail[2 * h + 1] << 8)) : (uint32_t)tail[h];
-      }
-    }
-  }
+  const int nr = p.num_tokens - j0 < R ? p.num_tokens - j0 : R;
+  const int64_t off = lane < nr ? row_offset(p, j0 + lane) : -1;
+  const int nch = p.rms_offset >> 3, npre = p.rms_offset & 7, nfull = nch >> 6, ns = nch & 63, heads = p.rms_heads;
+  const uint32_t ms = ns > 0 ? flat_mul(ns) : 0u, mh = heads > 0 ? flat_mul(heads) : 0u;
   const float sc = *p.scale;
+  uint16_t* out0 = reinterpret_cast<uint16_t*>(p.dst) + (int64_t)j0 * p.dst_stride;
+  // ---- loads ----
+  uint2 blk[R][NF], fl[R];
+  uint32_t tb[R], pre = 0u;
+  uint32_t flive = 0u, tlive = 0u;   // bit i: this lane's slot of pass i belongs to a row to write
 #pragma unroll
-  for (int i = 0; i < NQ; ++i) {
-    if (64 * i >= total) break;
+  for (int i = 0; i < R; ++i) {
+    const int64_t o = uniform64(off, i);
+    if (o < 0) continue;
+#pragma unroll
+    for (int k = 0; k < NF; ++k)
+      if (k < nfull) blk[i][k] = *reinterpret_cast<const uint2*>(p.cache + o + 8 * (lane + 64 * k));
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
     const int q = lane + 64 * i;
-    if (!(live & (1u << i))) continue;
-    const int r = (int)(__umul24((uint32_t)q, mq) >> 20);
-    const int c = q - (int)__umul24((uint32_t)r, (uint32_t)nel);
-    uint16_t* out = reinterpret_cast<uint16_t*>(p.dst) + (int64_t)(j0 + r) * p.dst_stride;
-    if (c < nch) {
-      const uint32_t w[2] = {raw[i].x, raw[i].y};
-      uint32_t o[4];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int wv = (int)w[h];
-        const float f0 = e4m3_f32(wv, 0) * sc, f1 = e4m3_f32(wv, 1) * sc;
-        const float f2 = e4m3_f32(wv, 2) * sc, f3 = e4m3_f32(wv, 3) * sc;
-        o[2 * h] = (uint32_t)to_out(f0, DT) | ((uint32_t)to_out(f1, DT) << 16);
-        o[2 * h + 1] = (uint32_t)to_out(f2, DT) | ((uint32_t)to_out(f3, DT) << 16);
+    if (64 * i < R * ns) {   // wave-uniform
+      const int r = q < nr * ns ? flat_row(q, ms) : 0;
+      const int64_t o = lane64(off, r);
+      if (q < nr * ns && o >= 0) {
+        flive |= 1u << i;
+        fl[i] = *reinterpret_cast<const uint2*>(p.cache + o + 512 * nfull + 8 * (q - r * ns));
       }
-      *reinterpret_cast<uint4*>(out + 8 * c) = make_uint4(o[0], o[1], o[2], o[3]);
-    } else {
-      // the 1-7 bytes between the last whole chunk and the rms tail (the plugin's rope-116 rows)
-      const uint32_t lo = (uint32_t)__shfl(roff_lo, r), hi = (uint32_t)__shfl(roff_hi, r);
-      const unsigned char* row = reinterpret_cast<const unsigned char*>(p.cache + (int64_t)(((uint64_t)hi << 32) | lo));
-      for (int e = 0; e < npre; ++e) out[c8 + e] = to_out(e4m3_f32((int)row[c8 + e], 0) * sc, DT);
+    }
+    if (64 * i < R * heads) {
+      const int r = q < nr * heads ? flat_row(q, mh) : 0;
+      const int64_t o = lane64(off, r);
+      if (q < nr * heads && o >= 0) {
+        tlive |= 1u << i;
+        const unsigned char* tail = reinterpret_cast<const unsigned char*>(p.cache + o) + p.rms_offset;
+        const int h = q - r * heads;
+        tb[i] = p.rms_mode == QMLA_RMS_BF16_BYTES ? ((uint32_t)tail[2 * h] | ((uint32_t)tail[2 * h + 1] << 8))
+                                                  : (uint32_t)tail[h];
+      }
     }
   }
-#pragma unroll
-  for (int i = 0; i < NT; ++i) {
-    if (64 * i >= nt) break;
-    const int t = lane + 64 * i;
-    const int r = (int)(__umul24((uint32_t)(t < nt ? t : 0), mt) >> 20);
-    const uint32_t lo = (uint32_t)__shfl(roff_lo, r), hi = (uint32_t)__shfl(roff_hi, r);
-    const int64_t ro = (int64_t)(((uint64_t)hi << 32) | lo);
-    if (t >= nt || ro < 0) continue;
-    const int h = t - (int)__umul24((uint32_t)r, (uint32_t)p.rms_heads);
-    uint16_t* out = reinterpret_cast<uint16_t*>(p.dst) + (int64_t)(j0 + r) * p.dst_stride + p.rms_offset;
-    float v;
-    if (p.rms_mode == QMLA_RMS_LOG8) {
-      v = l8[tb[i]];
-    } else if (p.rms_mode == QMLA_RMS_BF16_BYTES) {
-      if (DT == QMLA_DT_BF16) {
-        out[h] = (uint16_t)tb[i];
-        continue;
-      }
-      v = __uint_as_float(tb[i] << 16);
-    } else {
-      v = e4m3_f32((int)tb[i], 0) * sc;
-    }
-    out[h] = to_out(v, DT);
+  const int pr = npre > 0 ? lane / npre : R, pe = lane - pr * npre;   // this lane's pre-tail byte
+  bool plive = false;
+  if (npre > 0) {
+    const int64_t o = lane64(off, pr < nr ? pr : 0);
+    plive = pr < nr && o >= 0;
+    if (plive) pre = (uint32_t)(unsigned char)p.cache[o + 8 * nch + pe];
   }
+  // ---- conversions and stores ----
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    if (uniform64(off, i) < 0) continue;
+    uint16_t* out = out0 + i * p.dst_stride;
+#pragma unroll
+    for (int k = 0; k < NF; ++k)
+      if (k < nfull) *reinterpret_cast<uint4*>(out + 8 * (lane + 64 * k)) = dequant8<DT>(blk[i][k], sc);
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int q = lane + 64 * i;
+    if (flive & (1u << i)) {
+      const int r = flat_row(q, ms);
+      *reinterpret_cast<uint4*>(out0 + r * p.dst_stride + 512 * nfull + 8 * (q - r * ns)) = dequant8<DT>(fl[i], sc);
+    }
+    if (tlive & (1u << i)) {
+      const int r = flat_row(q, mh);
+      uint16_t* out = out0 + r * p.dst_stride + p.rms_offset + q - r * heads;
+      if (p.rms_mode == QMLA_RMS_LOG8) *out = to_out(kLog8.v[tb[i]], DT);
+      else if (p.rms_mode == QMLA_RMS_E4M3) *out = to_out(e4m3_f32((int)tb[i], 0) * sc, DT);
+      else *out = DT == QMLA_DT_BF16 ? (uint16_t)tb[i] : to_out(__uint_as_float(tb[i] << 16), DT);
+    }
+  }
+  if (plive) out0[pr * p.dst_stride + 8 * nch + pe] = to_out(e4m3_f32((int)pre, 0) * sc, DT);
 }
 
 }  // namespace ga
@@ -538,7 +607,7 @@ extern "C" int qmla_gather(const qmla_gather_params* p, void* stream) {
   k.cache = static_cast<const char*>(p->cache);
   k.page_stride = p->page_stride;
   k.token_stride = p->token_stride;
-  k.page_size = p->page_size;
+  k.page = page_div_of(p->page_size, (int64_t)p->bt_cols * p->page_size);
   k.num_pages = p->num_pages;
   k.kv_dtype = p->kv_dtype;
   k.rms_mode = p->rms_mode;
@@ -558,10 +627,14 @@ extern "C" int qmla_gather(const qmla_gather_params* p, void* stream) {
   k.dst_stride = p->dst_stride;
   k.dst_dtype = p->dst_dtype;
   void* args[] = {&k};
-  if (fp8 && p->num_tokens >= kMultiRowMin && p->rms_offset <= 1024 && p->rms_heads <= 64) {
-    const unsigned grid = (unsigned)((p->num_tokens + 4 * ga::GROWS - 1) / (4 * ga::GROWS));
-    const void* fn = p->dst_dtype == QMLA_DT_F16 ? (const void*)ga::gather_fp8_kernel<QMLA_DT_F16>
-                                                 : (const void*)ga::gather_fp8_kernel<QMLA_DT_BF16>;
+  if (fp8 && p->num_tokens >= kGatherRowsMin && p->rms_offset < 2048 && p->rms_heads <= 64) {
+    const bool wide = p->rms_offset >= 1024, f16 = p->dst_dtype == QMLA_DT_F16;
+    const int R = !wide && p->num_tokens >= kGatherRows4Min ? 4 : 2;
+    const unsigned grid = (unsigned)((p->num_tokens + 4 * R - 1) / (4 * R));
+#define QMLA_GA(RR, NF) \
+    (f16 ? (const void*)ga::gather_rows_kernel<QMLA_DT_F16, RR, NF> : (const void*)ga::gather_rows_kernel<QMLA_DT_BF16, RR, NF>)
+    const void* fn = wide ? QMLA_GA(2, 3) : R == 2 ? QMLA_GA(2, 1) : QMLA_GA(4, 1);
+#undef QMLA_GA
     const hipError_t e = hipLaunchKernel(fn, dim3(grid), dim3(256), args, 0, (hipStream_t)stream);
     return e == hipSuccess ? QMLA_OK : QMLA_ERR_LAUNCH;
   }
