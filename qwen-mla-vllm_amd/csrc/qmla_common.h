@@ -174,6 +174,7 @@ struct BalRange {
   int lo, hi;      // plan tiles of this workgroup
   int chunk, total;
   int b0, c0;      // the last request with C_b <= lo, and its C_b
+  int len[4];      // lane's lengths: request 64k + lane (0 past the last)
 };
 
 // One wave computes workgroup w's range (wave-uniform results; any wave may call it). The lengths of
@@ -187,6 +188,8 @@ __device__ inline BalRange balanced_range(const KParams& p, int w) {
   BalRange r;
   r.chunk = 1;
   r.lo = r.hi = r.total = r.b0 = r.c0 = 0;
+#pragma unroll
+  for (int k = 0; k < NK; ++k) r.len[k] = 0;
   if (p.n_req <= 0) return r;
   int t[NK], incl[NK];
 #pragma unroll
@@ -197,7 +200,8 @@ __device__ inline BalRange balanced_range(const KParams& p, int w) {
   int total = 0;
 #pragma unroll
   for (int k = 0; k < NK; ++k) {
-    t[k] = 64 * k + lane < p.n_req ? len_tiles<SW>(t[k]) : 0;
+    r.len[k] = 64 * k + lane < p.n_req ? t[k] : 0;
+    t[k] = len_tiles<SW>(r.len[k]);
     incl[k] = wave_incl_sum(t[k]);
     total += lane_value(incl[k], 63);
   }

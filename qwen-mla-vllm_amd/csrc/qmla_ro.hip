@@ -108,7 +108,7 @@ __device__ __forceinline__ float quad_bcast(float x) {
 
 template <class C, int ROLE>
 __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float kscale, bool fixed, int lo,
-                                          int hi, int b0, int c0, int wr, int& bad) {
+                                          int hi, int b0, int c0, int wr, const int (&len)[4], int& bad) {
   constexpr int NTHR = C::NTHR;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -264,7 +264,7 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
 
   for (;;) {
     if constexpr (ROLE == DMA) {
-      if (dw == 0) plan_window<kPlanSwitchRo>(p, sm, fixed, lo, hi, cb, ctok, cp);
+      if (dw == 0) plan_window<kPlanSwitchRo>(p, sm, fixed, lo, hi, cb, ctok, cp, len);
     }
     __syncthreads();
     const int nseg = sm.win[0], ntot = sm.win[1], npg = sm.win[2], more = sm.win[3];
@@ -573,7 +573,7 @@ __global__ __launch_bounds__(C::NTHR, 1) void ro_kernel(const KParams p) {
   const bool fixed = p.num_splits > 0;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = blockIdx.x;
-  int lo = 0, hi = 0, b0 = 0, c0 = 0;
+  int lo = 0, hi = 0, b0 = 0, c0 = 0, len[4] = {0, 0, 0, 0};
   if (!fixed) {
     if (wr == 0 && wv == C::NCW + 1) store_plan<kPlanSwitchRo>(p);   // for the balanced combine
     const BalRange r = balanced_range<kPlanSwitchRo>(p, wr);
@@ -581,12 +581,16 @@ __global__ __launch_bounds__(C::NTHR, 1) void ro_kernel(const KParams p) {
     hi = r.hi;
     b0 = r.b0;
     c0 = r.c0;
-    if (lo >= hi) return;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) len[k] = r.len[k];
   }
-  int bad = 0;
-  if (wv < C::NCW) role_main<C, COMPUTE>(p, sm, kscale, fixed, lo, hi, b0, c0, wr, bad);
-  else role_main<C, DMA>(p, sm, kscale, fixed, lo, hi, b0, c0, wr, bad);
-  report_pages(p, bad);
+  if (fixed || lo < hi) {
+    int bad = 0;
+    if (wv < C::NCW) role_main<C, COMPUTE>(p, sm, kscale, fixed, lo, hi, b0, c0, wr, len, bad);
+    else role_main<C, DMA>(p, sm, kscale, fixed, lo, hi, b0, c0, wr, len, bad);
+    report_pages(p, bad);
+  }
+  __builtin_amdgcn_wave_barrier();   // one exit for every path (no instruction)
 }
 
 typedef void (*RoFn)(const KParams);

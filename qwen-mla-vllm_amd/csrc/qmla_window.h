@@ -193,13 +193,15 @@ __device__ __forceinline__ void wait_tiles(int ahead) {
   }
 }
 
-// Wave 0: the next window of pieces, from request cb at token ctok on, into sm.seg / sm.win.
+// One wave: the next window of pieces, from request cb at token ctok on, into sm.seg / sm.win.
 // Lane l looks at request cb + l; pieces are taken in request order while their pages fit PN (the
 // first piece that does not fit is cut at a page boundary). Balanced mode: cp is the plan prefix
-// C_cb of the cursor's request, and the lanes' C_b follow from a scan of their tile counts.
+// C_cb of the cursor's request, and the lanes' C_b follow from a scan of their tile counts; len holds
+// the lengths of the first 256 requests as balanced_range loaded them (loaded again, they waited 1.7 us
+// behind the other waves' query loads at a workgroup's start).
 template <int SW, int PN = PIDN, class SM>
 __device__ void plan_window(const KParams& p, SM& sm, bool fixed, int lo, int hi, int& cb, int& ctok,
-                            int& cp) {
+                            int& cp, const int (&len)[4]) {
   const int lane = threadIdx.x & 63;
   const int P = p.page_size;
   int nseg = 0, ntot = 0, npg = 0;
@@ -207,8 +209,20 @@ __device__ void plan_window(const KParams& p, SM& sm, bool fixed, int lo, int hi
   while (more && nseg == 0) {
     const int b = cb + lane;
     int a = 0, e = 0, L = 0, fl = 0;
-    // plan tiles [c0, c1) of request b (balanced mode)
-    const int tb = (!fixed && b < p.n_req) ? plan_tiles<SW>(p, b) : 0;
+    // request b's length and its plan tiles [c0, c1) (balanced mode)
+    int Lb = 0;
+    if (!fixed) {
+      if (cb + 64 <= 256 || p.n_req <= 256) {
+        const int k = cb >> 6, at = (cb & 63) + lane;
+        const int l0 = k == 0 ? len[0] : k == 1 ? len[1] : k == 2 ? len[2] : k == 3 ? len[3] : 0;
+        const int l1 = k == 0 ? len[1] : k == 1 ? len[2] : k == 2 ? len[3] : 0;
+        const int x0 = __shfl(l0, at & 63), x1 = __shfl(l1, at & 63);
+        Lb = at < 64 ? x0 : x1;
+      } else if (b < p.n_req) {
+        Lb = req_len(p, b);
+      }
+    }
+    const int tb = len_tiles<SW>(Lb);
     const int tincl = wave_incl_sum(tb);
     const int c0 = cp + tincl - tb, c1 = cp + tincl;
     bool beyond;
@@ -227,7 +241,7 @@ __device__ void plan_window(const KParams& p, SM& sm, bool fixed, int lo, int hi
       if (!beyond) {
         beyond = c0 >= hi;
         if (!beyond && c1 > lo) {
-          L = req_len(p, b);
+          L = Lb;
           const PieceTok pt = piece_tokens<SW>(L, c0, c1, lo, hi);
           const int a0 = pt.a;
           e = pt.e;

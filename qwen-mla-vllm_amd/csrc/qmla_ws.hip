@@ -126,7 +126,8 @@ __device__ __forceinline__ constexpr int dpw(int d) { return (C::NI - d + C::NIW
 // registers live (score waves the query fragments, value waves the accumulators).
 template <class C, int ROLE>
 __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float kscale, bool fixed, int lo,
-                                          int hi, int b0, int c0, int wr, int hz, int& bad) {
+                                          int hi, int b0, int c0, int wr, int hz, const int (&len)[4],
+                                          int& bad) {
   constexpr int NTHR = C::NTHR;
   constexpr bool F8 = C::EB == 1;
   constexpr int NB = C::DCG / 128;       // latent blocks of the fp8 product
@@ -215,13 +216,14 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
     for (int k = 0; k < C::KQ; ++k) {
       const int col = !F8 ? 64 * (k >> 1) + 16 * lg + 8 * (k & 1)
                           : k < 4 * NB ? 128 * (k >> 2) + 32 * lg + 8 * (k & 3) : C::DCG + 16 * lg + 8 * (k - 4 * NB);
-      bf16x8 v = load_q8(col < C::DCG ? qnp + col : qpp + (col - C::DCG), p.q_vec);
-      if (!rok[m]) v = bf16x8{};
-      qn[k] = v;
+      qn[k] = load_q8(col < C::DCG ? qnp + col : qpp + (col - C::DCG), p.q_vec);
     }
   };
   // qn -> the MFMA operands of row block m
   auto set_q = [&](int m) {
+#pragma unroll
+    for (int k = 0; k < C::KQ; ++k)
+      if (!rok[m]) qn[k] = bf16x8{};
     if constexpr (F8) {
       float mx = 0.f;
 #pragma unroll
@@ -383,18 +385,17 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
 
   // window planning cursor (first value wave only): request, token, plan prefix of the request
   int cb = fixed ? (int)blockIdx.y : b0, ctok = 0, cp = c0;
-  // the range's first piece, if it has one, is the cursor's request: its query is loaded and converted
-  // while a value wave plans the window and the first tile is in flight, not in the first step
-  bool q_ready = false;
+  // the range's first piece, if it has one, is the cursor's request: its query is loaded while a value
+  // wave plans the window and converted while the first tile is in flight, not in the first step
+  bool q_ready = false, q_loaded = false;
   if constexpr (QS && C::G == 1) {
     load_q(cb, 0);
-    set_q(0);
-    q_ready = true;
+    q_loaded = true;
   }
 
   for (;;) {
     if constexpr (ROLE == VALUE) {
-      if (vw == 0) plan_window<kPlanSwitchWs>(p, sm, fixed, lo, hi, cb, ctok, cp);
+      if (vw == 0) plan_window<kPlanSwitchWs>(p, sm, fixed, lo, hi, cb, ctok, cp, len);
     }
     __syncthreads();
     const int nseg = sm.win[0], ntot = sm.win[1], npg = sm.win[2], more = sm.win[3];
@@ -413,6 +414,12 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
                                bad);
     }
     __syncthreads();
+
+    if constexpr (QS && C::G == 1) {
+      if (q_loaded) set_q(0);
+      q_ready = q_loaded;
+      q_loaded = false;
+    }
 
     // ---- per-role cursors over the window's pieces ----
     // DMA (value waves): piece ki, tile ti, page cursor (window page index ipg, token offset ioff)
@@ -906,7 +913,7 @@ __global__ __launch_bounds__(C::NTHR, 1) void ws_kernel(const KParams p) {
       wr = (int)blockIdx.x / p.hsplit;
     }
   }
-  int lo = 0, hi = 0, b0 = 0, c0 = 0;
+  int lo = 0, hi = 0, b0 = 0, c0 = 0, len[4] = {0, 0, 0, 0};
   if (!fixed) {
     if (wr == 0 && hz == 0 && wv == 5) store_plan<kPlanSwitchWs>(p);   // for the balanced combine
     const BalRange r = balanced_range<kPlanSwitchWs>(p, wr);
@@ -914,12 +921,16 @@ __global__ __launch_bounds__(C::NTHR, 1) void ws_kernel(const KParams p) {
     hi = r.hi;
     b0 = r.b0;
     c0 = r.c0;
-    if (lo >= hi) return;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) len[k] = r.len[k];
   }
-  int bad = 0;
-  if (wv < 4) role_main<C, SCORE>(p, sm, kscale, fixed, lo, hi, b0, c0, wr, hz, bad);
-  else role_main<C, VALUE>(p, sm, kscale, fixed, lo, hi, b0, c0, wr, hz, bad);
-  report_pages(p, bad);
+  if (fixed || lo < hi) {
+    int bad = 0;
+    if (wv < 4) role_main<C, SCORE>(p, sm, kscale, fixed, lo, hi, b0, c0, wr, hz, len, bad);
+    else role_main<C, VALUE>(p, sm, kscale, fixed, lo, hi, b0, c0, wr, hz, len, bad);
+    report_pages(p, bad);
+  }
+  __builtin_amdgcn_wave_barrier();   // one exit for every path (no instruction)
 }
 
 struct Inst {

@@ -144,7 +144,8 @@ __device__ __forceinline__ constexpr int dpw(int d) { return (C::NI - d + C::NIW
 // barrier sequence; each keeps only its own registers live.
 template <class C, int ROLE>
 __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float kscale, bool fixed, int lo, int hi,
-                                          int b0, int c0, int wr, int hz, int& bad) {
+                                          int b0, int c0, int wr, int hz, const int (&len)[4],
+                                          int& bad) {
   constexpr int NTHR = C::NTHR;
   constexpr bool QS = ROLE == SCORE;
   constexpr bool F8 = C::EB == 1;
@@ -342,7 +343,9 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
   // window planning cursor (first value wave only): request, token, plan prefix of the request
   int cb = fixed ? (int)blockIdx.y : b0, ctok = 0, cp = c0;
   // the range's first piece, if it has one, is the cursor's request: its query is loaded and converted
-  // while a value wave plans the window and the first tile is in flight, not in the first step
+  // while a value wave plans the window, not in the first step (converted after the plan, while the
+  // first tile is in flight, the loaded query is live across the window loop and spills 350 to 520
+  // bytes a lane in the fp8 instances)
   bool q_ready = false;
   if constexpr (QS) {
     load_q(cb);
@@ -351,7 +354,7 @@ __device__ __forceinline__ void role_main(const KParams& p, Smem<C>& sm, float k
 
   for (;;) {
     if constexpr (!QS) {
-      if (w == 0) plan_window<kPlanSwitchWs, PIDB>(p, sm, fixed, lo, hi, cb, ctok, cp);
+      if (w == 0) plan_window<kPlanSwitchWs, PIDB>(p, sm, fixed, lo, hi, cb, ctok, cp, len);
     }
     __syncthreads();
     const int nseg = sm.win[0], ntot = sm.win[1], npg = sm.win[2], more = sm.win[3];
@@ -748,7 +751,7 @@ __global__ __launch_bounds__(C::NTHR, 1) void wsb_kernel(const KParams p) {
       wr = (int)blockIdx.x / p.hsplit;
     }
   }
-  int lo = 0, hi = 0, b0 = 0, c0 = 0;
+  int lo = 0, hi = 0, b0 = 0, c0 = 0, len[4] = {0, 0, 0, 0};
   if (!fixed) {
     if (wr == 0 && hz == 0 && wv == 1) store_plan<kPlanSwitchWs>(p);   // for the balanced combine
     const BalRange r = balanced_range<kPlanSwitchWs>(p, wr);
@@ -756,12 +759,16 @@ __global__ __launch_bounds__(C::NTHR, 1) void wsb_kernel(const KParams p) {
     hi = r.hi;
     b0 = r.b0;
     c0 = r.c0;
-    if (lo >= hi) return;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) len[k] = r.len[k];
   }
-  int bad = 0;
-  if (wv >= 4) role_main<C, SCORE>(p, sm, kscale, fixed, lo, hi, b0, c0, wr, hz, bad);
-  else role_main<C, VALUE>(p, sm, kscale, fixed, lo, hi, b0, c0, wr, hz, bad);
-  report_pages(p, bad);
+  if (fixed || lo < hi) {
+    int bad = 0;
+    if (wv >= 4) role_main<C, SCORE>(p, sm, kscale, fixed, lo, hi, b0, c0, wr, hz, len, bad);
+    else role_main<C, VALUE>(p, sm, kscale, fixed, lo, hi, b0, c0, wr, hz, len, bad);
+    report_pages(p, bad);
+  }
+  __builtin_amdgcn_wave_barrier();   // one exit for every path (no instruction)
 }
 
 struct Inst {
