@@ -3,9 +3,10 @@
 //
 // Reference: qwen_mla/mla_impl.py:309-342 (QwenMLATritonImpl.do_kv_cache_update, the FP8 writer
 // with log8 or bf16-byte rms tails) and vLLM's concat_and_cache_mla for the rows the plugin hands
-// to it (bf16 caches; FP8 caches whose rms is e4m3). One wave per row: lane l converts latent
-// elements [8l, 8l+8) (and further 512-column blocks for wider latents), lanes 0.. the rope in 8s
-// and the rms tail one head each. Rows are independent, so the grid is rows / 4 workgroups of 256.
+// to it (bf16 caches; FP8 caches whose rms is e4m3). Up to a few thousand rows, and for bf16 caches,
+// one wave per row: lane l converts latent elements [8l, 8l+8) (and further 512-column blocks for wider
+// latents), lanes 0.. the rope in 8s and the rms tail one head each; more FP8 rows go two or four to a
+// wave (write_rows_kernel, gather_rows_kernel).
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
