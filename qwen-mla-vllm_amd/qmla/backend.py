@@ -140,7 +140,7 @@ def decode_params(impl, q, kv_c_and_k_pe_cache, attn_metadata, layer, out, lse):
                      out=out, lse=lse, d_c=rank, rope_w=rope_w, rms_offset=impl.rms_offset, rms_mode=rms_mode,
                      kv=kv, page_size=page_size, sm_scale=impl.scale, k_scale=k_scale,
                      qrows=1, groups=1, rms_heads=q_nope.shape[1], num_splits=0)
-    if q_pe is q_nope and rope_w > 0:
+    if not isinstance(q, tuple) and rope_w > 0:
         p.q_pe = q.data_ptr() + rank * q.element_size()
     if qrows > 1:
         p.qrows = fold_rows(p, qrows)

@@ -142,3 +142,14 @@ def test_decode_attention_fwd_refuses_a_host_scale():
     for ks in (0.5, torch.tensor(0.5, dtype=torch.float64)):
         with pytest.raises(TypeError, match="k_scale"):
             decode_attention_fwd(*args, k_scale=ks, is_mla=True, rms_offset=576, rms_log8=True)
+
+
+def test_decode_params_tuple_of_one_tensor():
+    """A tuple's parts are read as given, also where both are the same tensor."""
+    impl = QwenMLAHipImpl(kv_lora_rank=64, scale=0.1)
+    impl.rms_offset, impl.mla_local_heads, impl.mla_kv_fp8 = 128, 8, False
+    q = torch.zeros(3, 8, 64, dtype=torch.bfloat16)
+    cache = torch.zeros(5, 16, 144, dtype=torch.bfloat16)
+    p = decode_params(impl, (q, q), cache, _metadata(3), SimpleNamespace(), torch.empty_like(q), None)
+    assert p.q_nope == p.q_pe == q.data_ptr()
+    assert (p.q_pe_stride_row, p.q_pe_stride_head) == q.stride()[:2] and p.rope_w == 64
