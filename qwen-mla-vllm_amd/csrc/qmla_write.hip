@@ -157,7 +157,7 @@ __global__ __launch_bounds__(64 * ROWS_PER_WG) void write_kernel(const WParams p
     uint16_t* d16 = reinterpret_cast<uint16_t*>(dst);
     for (int c = 8 * lane; c < p.d_c; c += 512)
       *reinterpret_cast<uint4*>(d16 + c) = *reinterpret_cast<const uint4*>(kc + c);
-    const int pe = p.rope_w + (p.rms_mode == QMLA_RMS_BF16 ? p.rms_heads : 0);
+    const int pe = p.rope_w + p.rms_heads;
     for (int c = lane; c < pe; c += 64) d16[p.d_c + c] = kp[c];
   }
 }
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256) void write_rows_kernel(const WParams p) {
   if (r0 >= p.n) return;
   const int nr = p.n - r0 < R ? p.n - r0 : R;
   const int nfull = p.d_c >> 9, rem = (p.d_c >> 3) & 63, nrp = p.rope_w >> 3, npre = p.rope_w & 7;
-  const int ns = rem + nrp, heads = p.rms_mode == QMLA_RMS_NONE ? 0 : p.rms_heads;
+  const int ns = rem + nrp, heads = p.rms_heads;
   const uint32_t ms = ns > 0 ? flat_mul(ns) : 0u, mh = heads > 0 ? flat_mul(heads) : 0u;
   const uint16_t* kc = p.kv_c + (int64_t)r0 * p.kv_c_stride;
   const uint16_t* kp = p.k_pe + (int64_t)r0 * p.k_pe_stride;
@@ -298,7 +298,7 @@ extern "C" int qmla_cache_write(const qmla_cache_write_params* p, void* stream) 
   k.n = p->n;
   k.d_c = p->d_c;
   k.rope_w = p->rope_w;
-  k.rms_heads = p->rms_heads;
+  k.rms_heads = rb ? p->rms_heads : 0;   // without rms elements k_pe rows may end after the rope
   k.kv_dtype = p->kv_dtype;
   k.rms_mode = p->rms_mode;
   k.k_scale = p->k_scale;
@@ -308,7 +308,7 @@ extern "C" int qmla_cache_write(const qmla_cache_write_params* p, void* stream) 
   k.page = page_div_of(p->page_size, p->num_slots);
   k.num_slots = p->num_slots;
   void* args[] = {&k};
-  if (fp8 && p->n >= kWriteRowsMin && p->d_c <= 2047 && (p->d_c / 8) % 64 + p->rope_w / 8 <= 64 && p->rms_heads <= 64) {
+  if (fp8 && p->n >= kWriteRowsMin && p->d_c <= 2047 && (p->d_c / 8) % 64 + p->rope_w / 8 <= 64 && k.rms_heads <= 64) {
     constexpr int R = 2;
     const unsigned grid = (unsigned)((p->n + 4 * R - 1) / (4 * R));
     const void* fn = p->d_c < 1024 ? (const void*)wr::write_rows_kernel<R, 1> : (const void*)wr::write_rows_kernel<R, 3>;

@@ -38,6 +38,27 @@ def test_write(gpu, d_c, rope, heads, rms):
         assert torch.equal(got, want), (n, torch.nonzero(got != want)[:4])
 
 
+@pytest.mark.parametrize("kv", ["fp8", "bf16"])
+@pytest.mark.parametrize("n", [70, 2049])
+def test_write_without_rms_elements(gpu, kv, n):
+    """Rows without rms elements: k_pe is exactly the rope wide and exactly n rows long, whatever rms_heads
+    says (at both of the FP8 writer's row counts), and only latent and rope are written."""
+    import qmla
+    d_c, rope, heads = 512, 64, 24
+    g = torch.Generator(device="cuda").manual_seed(n)
+    kv_c = torch.randn(n, d_c, generator=g, device=gpu).to(torch.bfloat16)
+    k_pe = torch.randn(n, rope, generator=g, device=gpu).to(torch.bfloat16)
+    slots = torch.randperm(64 * 48, generator=torch.Generator().manual_seed(n))[:n].cuda()
+    cache = torch.full((64, 48, 608), 7, dtype=torch.uint8 if kv == "fp8" else torch.bfloat16, device=gpu)
+    qmla.cache_write(kv_c, k_pe, cache, slots, rope_w=rope, rms_heads=heads, kv_fp8=kv == "fp8", rms="none",
+                     k_scale=torch.ones((), device=gpu))
+    rows = cache.view(-1, 608)[slots]
+    want = torch.cat([kv_c, k_pe], -1)
+    if kv == "fp8":
+        want = want.float().clamp(-448, 448).to(torch.float8_e4m3fn).view(torch.uint8)
+    assert torch.equal(rows[:, :d_c + rope], want) and bool((rows[:, d_c + rope:] == 7).all())
+
+
 @pytest.mark.parametrize("rms", ["log8", "bf16", "e4m3"])
 @pytest.mark.parametrize("d_c,rope,heads", ROWS)
 def test_gather(gpu, d_c, rope, heads, rms):
