@@ -47,7 +47,8 @@ __device__ __forceinline__ int64_t uniform64(int64_t v, int lane) {   // lane's 
 // 3.2 us at one a wave, 3.3 at two; 4000 rows 4.5 and 3.9. Gather: 1000 rows 3.6 and 3.8, 12001 rows
 // 10.7 and 7.7 (rank 768: 12.1 and 9.8, rank 1792 16.9 and 15.1). Four rows a wave for rows below 1024
 // bytes: 20000 rows 10.9 and 10.5, 200000 rows 100 and 79 (rank 768: 131 and 128)
-constexpr int kWriteRowsMin = 2048, kGatherRowsMin = 4096, kGatherRows4Min = 16384;
+constexpr int kWriteRowsMin = 2048, kWriteRowsMin2 = 65536, kWriteWideMax = 131072;
+constexpr int kGatherRowsMin = 4096, kGatherRows4Min = 16384;
 namespace wr {
 
 constexpr int ROWS_PER_WG = 4;
@@ -164,21 +165,22 @@ __global__ __launch_bounds__(64 * ROWS_PER_WG) void write_kernel(const WParams p
 
 // FP8 rows: one wave writes R rows. Whole 512-column blocks of a row go one 8-column chunk to a lane
 // (row addresses in scalar registers); the chunks left over, the 1-7 rope elements before an rms tail
-// that is not 8-aligned, and the rms elements of the R rows are each dealt out flat over the wave.
-// Every load is in flight before the first conversion. The same bytes as write_kernel.
+// that is not 8-aligned, and the rms elements of the R rows are each dealt out flat over the wave (the
+// chunks in FP passes a row: up to 64 FP of them). Every load is in flight before the first conversion.
+// The same bytes as write_kernel.
 //
 // What bounds it: below some 20000 rows the launch of the waves and each one's chain of slot, row and
-// store, above that memory (60000 rows of rank 512: 108 MB in 21 us, 5.1 TB/s). 12001 rows of rank
-// 512 / 768 / 1792 at one row a wave 9.1 / 11.0 / 15.8 us (write_kernel), two rows 6.7 / 8.4 / 14.7,
-// four 6.6 / 9.0 / 16.7, eight 7.8 / 11.5 / 19.9; 200000 rows of rank 512 and 768, two rows 71 / 116,
-// four rows with every row's rope and tail passes of its own 75 / 115 (the form before this one).
-template <int R, int NF>
+// store, above that memory (65536 rows of rank 512: 118 MB in 23 us, 5.1 TB/s). 12001 rows of rank
+// 512 / 768 / 1792 at one row a wave 7.2 / 9.3 / 14.6 us (write_kernel), two rows 6.5 / 8.3 / 14.0,
+// four 6.4 / 8.6 / 16.5; 200000 rows of rank 512 and 768, one row 111 / 143, two 72 / 117, four 75 / 120.
+// The chunks' passes and the rms elements' in loops of their own: 65536 rows of rank 768 36.2 -> 32.0.
+template <int R, int NF, int FP>
 __global__ __launch_bounds__(256) void write_rows_kernel(const WParams p) {
   const int lane = threadIdx.x & 63;
   const int r0 = ((int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * R;
   if (r0 >= p.n) return;
   const int nr = p.n - r0 < R ? p.n - r0 : R;
-  const int nfull = p.d_c >> 9, rem = (p.d_c >> 3) & 63, nrp = p.rope_w >> 3, npre = p.rope_w & 7;
+  const int nch = p.d_c >> 3, nfull = nch >> 6, rem = nch & 63, nrp = p.rope_w >> 3, npre = p.rope_w & 7;
   const int ns = rem + nrp, heads = p.rms_heads;
   const uint32_t ms = ns > 0 ? flat_mul(ns) : 0u, mh = heads > 0 ? flat_mul(heads) : 0u;
   const uint16_t* kc = p.kv_c + (int64_t)r0 * p.kv_c_stride;
@@ -186,7 +188,7 @@ __global__ __launch_bounds__(256) void write_rows_kernel(const WParams p) {
   // ---- loads (rows past the end repeat the last row's) ----
   const int64_t slot0 = p.slots[r0 + (lane < nr ? lane : nr - 1)];
   const float inv = 1.0f / *p.k_scale;
-  uint4 lat[R][NF], fl[R];
+  uint4 lat[R][NF], fl[R * FP];
   uint16_t rm[R], pre = 0;
 #pragma unroll
   for (int i = 0; i < R; ++i) {
@@ -196,13 +198,17 @@ __global__ __launch_bounds__(256) void write_rows_kernel(const WParams p) {
       if (k < nfull) lat[i][k] = *reinterpret_cast<const uint4*>(row + 8 * (lane + 64 * k));
   }
 #pragma unroll
-  for (int i = 0; i < R; ++i) {
+  for (int i = 0; i < R * FP; ++i) {
     const int q = lane + 64 * i;
     if (64 * i < R * ns && q < nr * ns) {
       const int r = flat_row(q, ms), c = q - r * ns;
       fl[i] = *reinterpret_cast<const uint4*>(c < rem ? kc + r * p.kv_c_stride + 512 * nfull + 8 * c
                                                      : kp + r * p.k_pe_stride + 8 * (c - rem));
     }
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int q = lane + 64 * i;
     if (64 * i < R * heads && q < nr * heads) {
       const int r = flat_row(q, mh);
       rm[i] = kp[r * p.k_pe_stride + p.rope_w + q - r * heads];
@@ -226,15 +232,19 @@ __global__ __launch_bounds__(256) void write_rows_kernel(const WParams p) {
       if (k < nfull) *reinterpret_cast<uint2*>(p.cache + o + 8 * (lane + 64 * k)) = quant8r(lat[i][k], inv);
   }
 #pragma unroll
-  for (int i = 0; i < R; ++i) {
+  for (int i = 0; i < R * FP; ++i) {
     const int q = lane + 64 * i;
     if (64 * i < R * ns) {   // wave-uniform
       const int r = q < nr * ns ? flat_row(q, ms) : 0;
       const int64_t o = lane64(off, r);
       const int c = q - r * ns;
       if (q < nr * ns && o >= 0)
-        *reinterpret_cast<uint2*>(p.cache + o + 8 * (c < rem ? 64 * nfull + c : (p.d_c >> 3) + c - rem)) = quant8r(fl[i], inv);
+        *reinterpret_cast<uint2*>(p.cache + o + 8 * (c < rem ? 64 * nfull + c : nch + c - rem)) = quant8r(fl[i], inv);
     }
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int q = lane + 64 * i;
     if (64 * i < R * heads) {
       const int r = q < nr * heads ? flat_row(q, mh) : 0;
       const int64_t o = lane64(off, r);
@@ -257,6 +267,22 @@ __global__ __launch_bounds__(256) void write_rows_kernel(const WParams p) {
     if (pr < nr && o >= 0)
       p.cache[o + p.d_c + 8 * nrp + pe] = (char)(pack_e4m3(sat448(bf16_to_f32(pre), inv), 0.f, 0.f, 0.f) & 0xFF);
   }
+}
+
+// 8-column chunks of a row past its whole 512-column blocks
+static int flat_chunks(int d_c, int rope_w) { return (d_c / 8) % 64 + rope_w / 8; }
+
+// Which FP8 rows write_rows_kernel takes: up to 64 flat chunks a row (one pass), up to 128 below 1024
+// latent columns (two). Two passes pay once memory bounds the writer: d_c 448 with 128 rope columns, one
+// row a wave and two, 12001 rows 7.2 and 7.3 us, 65536 rows 29.7 and 25.0, 262144 rows 149 and 105 (768
+// with 264: 9.3 and 9.2, 36.3 and 35.3, 188 and 157; 256 with 512: 7.6 and 7.6, 30.5 and 28.6, 157 and
+// 134). From 1280 columns on they do so up to 131072 rows only (896 with 512: 65536 rows 52.4 and 44.9,
+// 131072 rows 114 and 118, 262144 rows 223 and 234).
+static bool several_rows(const qmla_cache_write_params* p, int ns, int heads) {
+  const bool two = ns > 64;
+  if (p->d_c >= 2048 || ns > (p->d_c < 1024 ? 128 : 64) || heads > 64) return false;
+  if (two && p->n >= kWriteWideMax && p->d_c + p->rope_w >= 1280) return false;
+  return p->n >= (two ? kWriteRowsMin2 : kWriteRowsMin);
 }
 
 }  // namespace wr
@@ -308,10 +334,13 @@ extern "C" int qmla_cache_write(const qmla_cache_write_params* p, void* stream) 
   k.page = page_div_of(p->page_size, p->num_slots);
   k.num_slots = p->num_slots;
   void* args[] = {&k};
-  if (fp8 && p->n >= kWriteRowsMin && p->d_c <= 2047 && (p->d_c / 8) % 64 + p->rope_w / 8 <= 64 && k.rms_heads <= 64) {
+  const int ns = wr::flat_chunks(p->d_c, p->rope_w);
+  if (fp8 && wr::several_rows(p, ns, k.rms_heads)) {
     constexpr int R = 2;
     const unsigned grid = (unsigned)((p->n + 4 * R - 1) / (4 * R));
-    const void* fn = p->d_c < 1024 ? (const void*)wr::write_rows_kernel<R, 1> : (const void*)wr::write_rows_kernel<R, 3>;
+    const void* fn = p->d_c >= 1024 ? (const void*)wr::write_rows_kernel<R, 3, 1>
+                     : ns > 64      ? (const void*)wr::write_rows_kernel<R, 1, 2>
+                                    : (const void*)wr::write_rows_kernel<R, 1, 1>;
     const hipError_t e = hipLaunchKernel(fn, dim3(grid), dim3(256), args, 0, (hipStream_t)stream);
     return e == hipSuccess ? QMLA_OK : QMLA_ERR_LAUNCH;
   }

@@ -38,6 +38,28 @@ def test_write(gpu, d_c, rope, heads, rms):
         assert torch.equal(got, want), (n, torch.nonzero(got != want)[:4])
 
 
+@pytest.mark.parametrize("d_c,rope,heads,rms", [(448, 128, 24, "log8"), (768, 264, 24, "e4m3"), (256, 512, 24, "bf16"),
+                                                (504, 516, 63, "log8"), (1016, 512, 64, "log8")])
+def test_write_two_chunk_passes(gpu, d_c, rope, heads, rms):
+    """Rows of more than 64 chunks besides their whole 512-column blocks: two passes over the wave, from
+    65536 rows on (d_c 1016 with rope 512 is the most a row can hold; 504 with 516 has a pre-tail)."""
+    import qmla
+    g = torch.Generator(device="cuda").manual_seed(d_c + rope)
+    width = -(-(d_c + rope + heads * (2 if rms == "bf16" else 1)) // 16) * 16
+    for n in (65535, 65537):
+        kv_c = (torch.randn(n, d_c, generator=g, device=gpu) * 200).to(torch.bfloat16)
+        k_pe = torch.exp(torch.randn(n, -(-(rope + heads) // 8) * 8, generator=g, device=gpu)).to(torch.bfloat16)
+        slots = torch.randperm(n, generator=torch.Generator().manual_seed(n)).cuda()
+        slots[n // 2] = 1 << 40                             # past the cache: skipped
+        got = torch.full((n // 48 + 1, 48, width), 0xAB, dtype=torch.uint8, device=gpu)
+        want = got.clone()
+        kw = dict(rope_w=rope, rms_heads=heads, kv_fp8=True, rms=rms, k_scale=torch.tensor(0.37, device=gpu))
+        qmla.cache_write(kv_c, k_pe, got, slots, **kw)
+        for a in range(0, n, 1900):
+            qmla.cache_write(kv_c[a:], k_pe[a:], want, slots[a:a + 1900], **kw)
+        assert torch.equal(got, want), (n, torch.nonzero(got != want)[:4])
+
+
 @pytest.mark.parametrize("kv", ["fp8", "bf16"])
 @pytest.mark.parametrize("n", [70, 2049])
 def test_write_without_rms_elements(gpu, kv, n):
