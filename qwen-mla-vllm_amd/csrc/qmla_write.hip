@@ -43,11 +43,12 @@ __device__ __forceinline__ int64_t uniform64(int64_t v, int lane) {   // lane's 
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)v >> 32), lane);
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
-// rows from which FP8 rows are written and gathered several to a wave. Writer: 1000 rows of rank 512
-// 3.2 us at one a wave, 3.3 at two; 4000 rows 4.5 and 3.9. Gather: 1000 rows 3.6 and 3.8, 12001 rows
+// rows from which FP8 rows are written and gathered several to a wave. Writer, rank 512 / 768 / 1792:
+// 2048 rows 3.1 / 3.4 / 4.2 us at one a wave, 3.3 / 3.5 / 4.5 at two; 3000 rows 3.5 / 4.0 / 5.0 and 3.6 /
+// 4.1 / 5.3; 4096 rows 4.0 / 4.6 / 5.9 and 3.7 / 4.2 / 5.7. Gather: 1000 rows 3.6 and 3.8, 12001 rows
 // 10.7 and 7.7 (rank 768: 12.1 and 9.8, rank 1792 16.9 and 15.1). Four rows a wave for rows below 1024
 // bytes: 20000 rows 10.9 and 10.5, 200000 rows 100 and 79 (rank 768: 131 and 128)
-constexpr int kWriteRowsMin = 2048, kWriteRowsMin2 = 65536, kWriteWideMax = 131072;
+constexpr int kWriteRowsMin = 4096, kWriteRowsMin2 = 65536, kWriteWideMax = 131072;
 constexpr int kGatherRowsMin = 4096, kGatherRows4Min = 16384;
 namespace wr {
 
@@ -277,11 +278,14 @@ static int flat_chunks(int d_c, int rope_w) { return (d_c / 8) % 64 + rope_w / 8
 // row a wave and two, 12001 rows 7.2 and 7.3 us, 65536 rows 29.7 and 25.0, 262144 rows 149 and 105 (768
 // with 264: 9.3 and 9.2, 36.3 and 35.3, 188 and 157; 256 with 512: 7.6 and 7.6, 30.5 and 28.6, 157 and
 // 134). From 1280 columns on they do so up to 131072 rows only (896 with 512: 65536 rows 52.4 and 44.9,
-// 131072 rows 114 and 118, 262144 rows 223 and 234).
+// 131072 rows 114 and 118, 262144 rows 223 and 234). One pass: from 1408 columns on up to 131072 rows only
+// (rank 1792 with 232: 65536 rows 79.0 at one row a wave and 78.7 at two, 131072 rows 151 and 155, 262144
+// rows 292 and 309; 1536 with 128: 66.0 and 64.6, 135 and 138, 266 and 277; 1280 with 64: 262144 rows 231
+// and 229).
 static bool several_rows(const qmla_cache_write_params* p, int ns, int heads) {
   const bool two = ns > 64;
   if (p->d_c >= 2048 || ns > (p->d_c < 1024 ? 128 : 64) || heads > 64) return false;
-  if (two && p->n >= kWriteWideMax && p->d_c + p->rope_w >= 1280) return false;
+  if (p->n >= kWriteWideMax && p->d_c + p->rope_w >= (two ? 1280 : 1408)) return false;
   return p->n >= (two ? kWriteRowsMin2 : kWriteRowsMin);
 }
 
