@@ -19,7 +19,7 @@ def test_write(gpu, d_c, rope, heads, rms):
     import qmla
     g = torch.Generator(device="cuda").manual_seed(d_c + rope)
     width = -(-(d_c + rope + heads * {"bf16": 2, "none": 0}.get(rms, 1)) // 16) * 16
-    for n in (2047, 2048, 2049, 2055, 5003):
+    for n in (2047, 2048, 2049, 2055, 4095, 4096, 4097, 4103, 5003):
         pages, page = n // 48 + 2, 48
         kv_c = (torch.randn(n + 1, d_c, generator=g, device=gpu) * 200).to(torch.bfloat16)
         pe_w = -(-(rope + heads) // 8) * 8
@@ -61,7 +61,7 @@ def test_write_two_chunk_passes(gpu, d_c, rope, heads, rms):
 
 
 @pytest.mark.parametrize("kv", ["fp8", "bf16"])
-@pytest.mark.parametrize("n", [70, 2049])
+@pytest.mark.parametrize("n", [70, 4097])
 def test_write_without_rms_elements(gpu, kv, n):
     """Rows without rms elements: k_pe is exactly the rope wide and exactly n rows long, whatever rms_heads
     says (at both of the FP8 writer's row counts), and only latent and rope are written."""
@@ -70,8 +70,8 @@ def test_write_without_rms_elements(gpu, kv, n):
     g = torch.Generator(device="cuda").manual_seed(n)
     kv_c = torch.randn(n, d_c, generator=g, device=gpu).to(torch.bfloat16)
     k_pe = torch.randn(n, rope, generator=g, device=gpu).to(torch.bfloat16)
-    slots = torch.randperm(64 * 48, generator=torch.Generator().manual_seed(n))[:n].cuda()
-    cache = torch.full((64, 48, 608), 7, dtype=torch.uint8 if kv == "fp8" else torch.bfloat16, device=gpu)
+    slots = torch.randperm(96 * 48, generator=torch.Generator().manual_seed(n))[:n].cuda()
+    cache = torch.full((96, 48, 608), 7, dtype=torch.uint8 if kv == "fp8" else torch.bfloat16, device=gpu)
     qmla.cache_write(kv_c, k_pe, cache, slots, rope_w=rope, rms_heads=heads, kv_fp8=kv == "fp8", rms="none",
                      k_scale=torch.ones((), device=gpu))
     rows = cache.view(-1, 608)[slots]
