@@ -45,11 +45,10 @@ __device__ __forceinline__ int64_t uniform64(int64_t v, int lane) {   // lane's 
 }
 // rows from which FP8 rows are written and gathered several to a wave. Writer, rank 512 / 768 / 1792:
 // 2048 rows 3.1 / 3.4 / 4.2 us at one a wave, 3.3 / 3.5 / 4.5 at two; 3000 rows 3.5 / 4.0 / 5.0 and 3.6 /
-// 4.1 / 5.3; 4096 rows 4.0 / 4.6 / 5.9 and 3.7 / 4.2 / 5.7. Gather: 1000 rows 3.6 and 3.8, 12001 rows
-// 10.7 and 7.7 (rank 768: 12.1 and 9.8, rank 1792 16.9 and 15.1). Four rows a wave for rows below 1024
-// bytes: 20000 rows 10.9 and 10.5, 200000 rows 100 and 79 (rank 768: 131 and 128)
+// 4.1 / 5.3; 4096 rows 4.0 / 4.6 / 5.9 and 3.7 / 4.2 / 5.7. Gather: 4096 rows 4.8 / 5.2 / 7.4 and 4.5 /
+// 5.4 / 7.9, 12001 rows 9.2 / 9.6 / 14.4 and 7.6 / 9.2 / 14.2
 constexpr int kWriteRowsMin = 4096, kWriteRowsMin2 = 65536, kWriteWideMax = 131072;
-constexpr int kGatherRowsMin = 4096, kGatherRows4Min = 16384;
+constexpr int kGatherRowsMin = 4096;
 namespace wr {
 
 constexpr int ROWS_PER_WG = 4;
@@ -523,9 +522,9 @@ __device__ __forceinline__ uint4 dequant8(const uint2 raw, float sc) {
 // first conversion. The same values as gather_kernel.
 //
 // What bounds it: as write_rows_kernel, the waves and their chain (sequence, page, row) below some 20000
-// rows, memory above. 20000 rows of rank 512 / 768 / 1792: 16.1 / 17.4 / 24.6 us at one row a wave with
-// a 64-bit division and an exp2 in double for each, 10.9 / 14.2 / 21.7 at two rows, 10.5 / 14.7 / 22.8
-// at four; 60000 rows 39 / 41 / 82 at one, 24.4 / 32.0 / 76 at two, 22.7 / 32.6 / 86 at four.
+// rows, memory above. 20000 rows of rank 512 / 768 / 1792: 13.4 / 14.3 / 21.6 us at one row a wave
+// (gather_kernel), 11.0 / 13.5 / 20.7 at two rows, 10.6 / 14.7 / 23.6 at four; 65536 rows 34.8 / 35.9 /
+// 59.6 at one, 26.5 / 35.1 / 62.2 at two, 24.2 / 34.9 / 65.7 at four.
 template <int DT, int R, int NF>
 __global__ __launch_bounds__(256) void gather_rows_kernel(const GParams p) {
   const int lane = threadIdx.x & 63;
@@ -606,6 +605,19 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const GParams p) {
   if (plive) out0[pr * p.dst_stride + 8 * nch + pe] = to_out(e4m3_f32((int)pre, 0) * sc, DT);
 }
 
+// Rows a wave of gather_rows_kernel, two or four. Below 1024 columns four pay from 16384 rows on where the
+// rows' flat chunks then fit fewer passes each (576 columns 65536 rows 26.5 us at two and 24.2 at four; 884:
+// 16384 rows 12.4 and 11.7, 65536 rows 35.3 and 31.6), and from 32768 rows on where they do not (1000
+// columns, 61 chunks: 16384 rows 12.3 and 13.0, 30000 rows 18.5 and 19.4, 65536 rows 35.1 and 34.9, 200000
+// rows 120 and 105; 704 columns: 30000 rows 15.5 and 16.2, 200000 rows 79 and 75), and never at rank 1792
+// (200000 rows 209 and 232).
+static int rows_per_wave(const qmla_gather_params* p) {
+  const int n = p->num_tokens, ns = p->rms_offset / 8 % 64;
+  if (p->rms_offset >= 1024) return 2;
+  const bool fewer = (4 * ns + 63) / 64 < 2 * ((2 * ns + 63) / 64);
+  return n >= (fewer ? 16384 : 32768) ? 4 : 2;
+}
+
 }  // namespace ga
 }  // namespace qmla
 
@@ -663,7 +675,7 @@ extern "C" int qmla_gather(const qmla_gather_params* p, void* stream) {
   void* args[] = {&k};
   if (fp8 && p->num_tokens >= kGatherRowsMin && p->rms_offset < 2048 && p->rms_heads <= 64) {
     const bool wide = p->rms_offset >= 1024, f16 = p->dst_dtype == QMLA_DT_F16;
-    const int R = !wide && p->num_tokens >= kGatherRows4Min ? 4 : 2;
+    const int R = ga::rows_per_wave(p);
     const unsigned grid = (unsigned)((p->num_tokens + 4 * R - 1) / (4 * R));
 #define QMLA_GA(RR, NF) \
     (f16 ? (const void*)ga::gather_rows_kernel<QMLA_DT_F16, RR, NF> : (const void*)ga::gather_rows_kernel<QMLA_DT_BF16, RR, NF>)

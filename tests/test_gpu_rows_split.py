@@ -81,30 +81,41 @@ def test_write_without_rms_elements(gpu, kv, n):
     assert torch.equal(rows[:, :d_c + rope], want) and bool((rows[:, d_c + rope:] == 7).all())
 
 
+def _check_gather(gpu, d_c, rope, heads, rms, n, step):
+    import qmla
+    lens = [1, n // 3, n - 1 - n // 3 - 7, 7]
+    c = make_case(batch=4, heads=heads, d_c=d_c, rope_w=rope, page_size=48, lens=lens, kv="fp8",
+                  rms_mode="bf16_bytes" if rms == "bf16" else rms, seed=n, device=gpu, rms="spread", amp=4.0)
+    c.cache.view(torch.uint8).view(-1)[:2048] = torch.arange(2048, device=gpu).to(torch.uint8) & 0x8F   # small, -0
+    table = c.block_table.clone()
+    table[1, 5] = c.cache.shape[0] + 9                  # a page outside the cache: its rows are skipped
+    t = torch.tensor(lens)
+    cu = torch.cat([torch.zeros(1, dtype=torch.int64), t.cumsum(0)]).to(torch.int32).cuda()
+    seq = torch.repeat_interleave(torch.arange(4, dtype=torch.int32), t).cuda()
+    for dtype in (torch.bfloat16, torch.float16):
+        got = torch.full((n + 2, c.row), 7.0, dtype=dtype, device=gpu)
+        want = got.clone()
+
+        def gather(dst, a, m):
+            qmla.gather_cache(src_cache=c.cache[:, :, 0, :], dst=dst[a:a + m], block_table=table,
+                              cu_seq_lens=cu - a, token_to_seq=seq[a:a + m], num_tokens=m, kv_cache_dtype="fp8",
+                              scale=c.k_scale, mla_rms=(c.rms_offset, heads, rms))
+
+        gather(got, 0, n)
+        for a in range(0, n, step):
+            gather(want, a, min(step, n - a))
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (n, dtype)
+
+
 @pytest.mark.parametrize("rms", ["log8", "bf16", "e4m3"])
 @pytest.mark.parametrize("d_c,rope,heads", ROWS)
 def test_gather(gpu, d_c, rope, heads, rms):
-    import qmla
     for n in (4095, 4096, 4101) + ((16383, 16384, 16387) if rms == "log8" else ()):
-        lens = [1, n // 3, n - 1 - n // 3 - 7, 7]
-        c = make_case(batch=4, heads=heads, d_c=d_c, rope_w=rope, page_size=48, lens=lens, kv="fp8",
-                      rms_mode="bf16_bytes" if rms == "bf16" else rms, seed=n, device=gpu, rms="spread", amp=4.0)
-        c.cache.view(torch.uint8).view(-1)[:2048] = torch.arange(2048, device=gpu).to(torch.uint8) & 0x8F   # small, -0
-        table = c.block_table.clone()
-        table[1, 5] = c.cache.shape[0] + 9                  # a page outside the cache: its rows are skipped
-        t = torch.tensor(lens)
-        cu = torch.cat([torch.zeros(1, dtype=torch.int64), t.cumsum(0)]).to(torch.int32).cuda()
-        seq = torch.repeat_interleave(torch.arange(4, dtype=torch.int32), t).cuda()
-        for dtype in (torch.bfloat16, torch.float16):
-            got = torch.full((n + 2, c.row), 7.0, dtype=dtype, device=gpu)
-            want = got.clone()
+        _check_gather(gpu, d_c, rope, heads, rms, n, 1000)
 
-            def gather(dst, a, m):
-                qmla.gather_cache(src_cache=c.cache[:, :, 0, :], dst=dst[a:a + m], block_table=table,
-                                  cu_seq_lens=cu - a, token_to_seq=seq[a:a + m], num_tokens=m, kv_cache_dtype="fp8",
-                                  scale=c.k_scale, mla_rms=(c.rms_offset, heads, rms))
 
-            gather(got, 0, n)
-            for a in range(0, n, 1000):
-                gather(want, a, min(1000, n - a))
-            assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (n, dtype)
+@pytest.mark.parametrize("d_c,rope,heads,n", [(768, 232, 24, 32769), (640, 64, 24, 32770), (448, 64, 64, 32771)])
+def test_gather_four_rows_a_wave(gpu, d_c, rope, heads, n):
+    """Four rows a wave where the line lies higher: flat chunks that fill two rows' passes, and no flat
+    chunks at all."""
+    _check_gather(gpu, d_c, rope, heads, "log8", n, 4000)
