@@ -609,11 +609,12 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const GParams p) {
 // rows' flat chunks then fit fewer passes each (576 columns 65536 rows 26.5 us at two and 24.2 at four; 884:
 // 16384 rows 12.4 and 11.7, 65536 rows 35.3 and 31.6), and from 32768 rows on where they do not (1000
 // columns, 61 chunks: 16384 rows 12.3 and 13.0, 30000 rows 18.5 and 19.4, 65536 rows 35.1 and 34.9, 200000
-// rows 120 and 105; 704 columns: 30000 rows 15.5 and 16.2, 200000 rows 79 and 75), and never at rank 1792
-// (200000 rows 209 and 232).
+// rows 120 and 105; 704 columns: 30000 rows 15.5 and 16.2, 200000 rows 79 and 75). Up to 1280 columns four
+// pay once the rows and their copies outgrow the memory-side cache (1024 columns: 131072 rows 63.7 and
+// 66.2, 160000 rows 88 and 81, 262144 rows 157 and 138), and never at rank 1792 (200000 rows 209 and 232).
 static int rows_per_wave(const qmla_gather_params* p) {
   const int n = p->num_tokens, ns = p->rms_offset / 8 % 64;
-  if (p->rms_offset >= 1024) return 2;
+  if (p->rms_offset >= 1024) return p->rms_offset <= 1280 && n >= 150000 ? 4 : 2;
   const bool fewer = (4 * ns + 63) / 64 < 2 * ((2 * ns + 63) / 64);
   return n >= (fewer ? 16384 : 32768) ? 4 : 2;
 }
@@ -679,7 +680,7 @@ extern "C" int qmla_gather(const qmla_gather_params* p, void* stream) {
     const unsigned grid = (unsigned)((p->num_tokens + 4 * R - 1) / (4 * R));
 #define QMLA_GA(RR, NF) \
     (f16 ? (const void*)ga::gather_rows_kernel<QMLA_DT_F16, RR, NF> : (const void*)ga::gather_rows_kernel<QMLA_DT_BF16, RR, NF>)
-    const void* fn = wide ? QMLA_GA(2, 3) : R == 2 ? QMLA_GA(2, 1) : QMLA_GA(4, 1);
+    const void* fn = wide ? (R == 2 ? QMLA_GA(2, 3) : QMLA_GA(4, 3)) : R == 2 ? QMLA_GA(2, 1) : QMLA_GA(4, 1);
 #undef QMLA_GA
     const hipError_t e = hipLaunchKernel(fn, dim3(grid), dim3(256), args, 0, (hipStream_t)stream);
     return e == hipSuccess ? QMLA_OK : QMLA_ERR_LAUNCH;

@@ -114,8 +114,9 @@ def test_gather(gpu, d_c, rope, heads, rms):
         _check_gather(gpu, d_c, rope, heads, rms, n, 1000)
 
 
-@pytest.mark.parametrize("d_c,rope,heads,n", [(768, 232, 24, 32769), (640, 64, 24, 32770), (448, 64, 64, 32771)])
+@pytest.mark.parametrize("d_c,rope,heads,n", [(768, 232, 24, 32769), (640, 64, 24, 32770), (448, 64, 64, 32771),
+                                              (960, 64, 24, 150001), (1024, 116, 12, 150003)])
 def test_gather_four_rows_a_wave(gpu, d_c, rope, heads, n):
-    """Four rows a wave where the line lies higher: flat chunks that fill two rows' passes, and no flat
-    chunks at all."""
+    """Four rows a wave where the line lies higher: flat chunks that fill two rows' passes, no flat chunks
+    at all, and rows of 1024 columns and more (with and without a tail at 4 mod 8)."""
     _check_gather(gpu, d_c, rope, heads, "log8", n, 4000)
