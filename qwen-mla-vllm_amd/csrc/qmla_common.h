@@ -64,17 +64,19 @@ struct KParams {
                         // |value| <= 448), which the combine applies; else fp32
 };
 
-// x / d = (x * mul) >> sh for 0 <= x < 2^31: sh = 31 + ceil(log2 d), mul = ceil(2^sh / d) < 2^32, so
-// mul exceeds 2^sh / d by less than one part in 2^31 * d / 2^sh.
+// x / d = (x * mul) >> sh for 0 <= x < 2^31, 1 <= d < 2^31: sh = 31 + ceil(log2 d), mul = ceil(2^sh / d) <
+// 2^32. With e = mul * d - 2^sh < d <= 2^(sh - 31), x * mul / 2^sh = x/d + (x * e) / (d * 2^sh) lies less
+// than 1/d above x/d, so both have the same integer part.
 inline void page_magic(int d, uint32_t& mul, int& sh) {
   int l = 0;
   while (((int64_t)1 << l) < d) ++l;
   sh = 31 + l;
   mul = (uint32_t)((((uint64_t)1 << sh) + (uint64_t)d - 1) / (uint64_t)d);
 }
-__device__ __forceinline__ int page_div(const KParams& p, int x) {
-  return (int)(((uint64_t)(uint32_t)x * p.page_mul) >> p.page_sh);
+__host__ __device__ __forceinline__ uint32_t magic_div(uint32_t x, uint32_t mul, int sh) {
+  return (uint32_t)(((uint64_t)x * mul) >> sh);
 }
+__device__ __forceinline__ int page_div(const KParams& p, int x) { return (int)magic_div((uint32_t)x, p.page_mul, p.page_sh); }
 
 // A block-table entry checked against the page bound: an entry outside [0, page_bound) reads page 0
 // (in bounds) and raises `bad`, which the kernel reports once its memory traffic has drained.

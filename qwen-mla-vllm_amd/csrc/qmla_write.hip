@@ -28,7 +28,7 @@ static PageDiv page_div_of(int page_size, int64_t tokens) {
   return d;
 }
 __device__ __forceinline__ int64_t page_of(const PageDiv& d, int64_t tok) {
-  return d.mul ? (int64_t)(((uint64_t)(uint32_t)tok * d.mul) >> d.sh) : tok / d.size;
+  return d.mul ? (int64_t)magic_div((uint32_t)tok, d.mul, d.sh) : tok / d.size;
 }
 // flat slots of a wave's rows: slot q of rows of n slots is slot (q - r n) of row r = q / n, from a
 // 24-bit multiplication (q < 2^10, exact below 2^20 / n)
