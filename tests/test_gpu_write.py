@@ -119,6 +119,27 @@ def test_log8_codes_edges(gpu):
     assert np.array_equal(got[:n, D_C + ROPE:D_C + ROPE + H], exp[:, D_C + ROPE:])
 
 
+@pytest.mark.parametrize("copies", [1, 4])
+def test_log8_code_of_every_bf16(gpu, copies):
+    """Every bf16 value that is a number (infinities, zeros, negatives and subnormals among them) as an rms
+    element: the oracle's code, in the kernels of one row and of several rows a wave (5464 rows)."""
+    import qmla
+    bits = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    vals = bits[~torch.isnan(bits)]
+    n = -(-vals.numel() // 48)
+    rms = torch.ones(n * 48, dtype=torch.bfloat16)
+    rms[:vals.numel()] = vals
+    rms = rms.view(n, 48)
+    kv_c, k_pe = torch.zeros(n, 64, dtype=torch.bfloat16), torch.cat([torch.zeros(n, 8, dtype=torch.bfloat16), rms], 1)
+    N = copies * n
+    cache = torch.zeros(N // 16 + 1, 16, 128, dtype=torch.uint8, device=gpu)
+    qmla.cache_write(kv_c.repeat(copies, 1).to(gpu), k_pe.repeat(copies, 1).to(gpu), cache, torch.arange(N, device=gpu),
+                     rope_w=8, rms_heads=48, kv_fp8=True, rms="log8", k_scale=torch.ones((), device=gpu))
+    exp = ora.log8_encode(rms.float().numpy())
+    got = cache.cpu().view(-1, 128).numpy()[:N, 72:120]
+    assert np.array_equal(got, np.tile(exp, (copies, 1)))
+
+
 def test_bf16_rows_copied(gpu):
     import qmla
     n, P, pages = 50, 16, 10
