@@ -862,7 +862,8 @@ __global__ __launch_bounds__(64 * (SPLIT ? CM_MW : CM_AW)) void combine_bal_kern
 #pragma unroll
   for (int c = 0; c < NC; ++c) a[c] = 0.f;
   const int lc = col < dv ? col : 0, rl = jq * p.heads + head;
-  // rows of whole lane vectors (every compiled layout), else element loads
+  // rows of whole lane vectors (every layout a decode kernel is compiled for), else element loads: the
+  // combine entry point takes partials of any even width
   if (dv % NC == 0) merge_segments<H, NC, true>(p, (int64_t)w0 + req, rl, dv, lc, sub, split, nseg, m, l, a);
   else merge_segments<H, NC, false>(p, (int64_t)w0 + req, rl, dv, lc, sub, split, nseg, m, l, a);
   if constexpr (!SPLIT) {
@@ -1243,7 +1244,7 @@ static int run_empty_rows(const qmla_decode_params* p, KParams& k, hipStream_t s
 static int run_combine(const qmla_decode_params* p, KParams& k, hipStream_t st) {
   int dv = p->d_c / p->groups;
   void* args[] = {&k, &dv};
-  if (p->num_splits == 0 && (dv & 1)) return QMLA_ERR_SHAPE;   // the balanced combine reads column pairs
+  if (p->num_splits == 0 && (dv & 1)) return QMLA_ERR_SHAPE;   // no row format has an odd number of columns
   if (p->num_splits == 0) {
     // columns a lane and chunks of columns per (row, head); a chunk is split over up to 8 waves while
     // they stay within 2048, 8 a CU (23 rank-768 requests, 1104 chunks: 7.9 us unsplit, 10.8 split
