@@ -826,8 +826,12 @@ __device__ __forceinline__ void merge_segments(const KParams& p, int64_t slot0, 
 
 // H = fp16 partials without the fp8 scale, which is applied here; nch chunks of 64*NC columns per
 // row; `split` waves per chunk (1 unless SPLIT). Workgroups of nch*split waves (SPLIT: one head), or
-// of CM_AW waves that take the chunks of CM_AW / nch heads.
-template <bool H, int NC, bool SPLIT>
+// of CM_AW waves that take the chunks of CM_AW / nch heads. VEC: rows of whole lane vectors, as every
+// layout a decode kernel is compiled for; the combine entry point takes partials of any even width, which
+// are read by elements. Those loads in the same kernel took it from 43-94 VGPRs to 77-138, at 3 waves a
+// SIMD instead of 5 to 8, for rows that never use them: 700 rank-1792 bf16 requests of 150 tokens 33.0 us
+// with them and 28.0 without, 128 of 1500 17.3 / 15.2, 128 rank-1792 fp8 requests of 6000 17.5 / 14.2.
+template <bool H, int NC, bool SPLIT, bool VEC>
 __global__ __launch_bounds__(64 * (SPLIT ? CM_MW : CM_AW)) void combine_bal_kernel(const KParams p, int dv, int nch, int split) {
   constexpr int CW = 64 * NC;
   const int row = blockIdx.y;
@@ -862,10 +866,7 @@ __global__ __launch_bounds__(64 * (SPLIT ? CM_MW : CM_AW)) void combine_bal_kern
 #pragma unroll
   for (int c = 0; c < NC; ++c) a[c] = 0.f;
   const int lc = col < dv ? col : 0, rl = jq * p.heads + head;
-  // rows of whole lane vectors (every layout a decode kernel is compiled for), else element loads: the
-  // combine entry point takes partials of any even width
-  if (dv % NC == 0) merge_segments<H, NC, true>(p, (int64_t)w0 + req, rl, dv, lc, sub, split, nseg, m, l, a);
-  else merge_segments<H, NC, false>(p, (int64_t)w0 + req, rl, dv, lc, sub, split, nseg, m, l, a);
+  merge_segments<H, NC, VEC>(p, (int64_t)w0 + req, rl, dv, lc, sub, split, nseg, m, l, a);
   if constexpr (!SPLIT) {
     const float inv = inv_sum(osc, l);
 #pragma unroll
@@ -1249,17 +1250,20 @@ static int run_combine(const qmla_decode_params* p, KParams& k, hipStream_t st) 
     // columns a lane and chunks of columns per (row, head); a chunk is split over up to 8 waves while
     // they stay within 2048, 8 a CU (23 rank-768 requests, 1104 chunks: 7.9 us unsplit, 10.8 split
     // over 4; bf16 B 4, 96 chunks: 4.3 split over 8, 7.2 unsplit)
-    const int nc = dv <= 256 ? 4 : 8;
+    const int nc = dv <= 256 && dv % 4 == 0 ? 4 : 8;
+    const bool vec = dv % nc == 0;
     int nch = (dv + 64 * nc - 1) / (64 * nc), split = 1;
     const int64_t chunks = (int64_t)p->rows * p->heads * nch;
-    while (2 * split * nch <= CM_MW && chunks * 2 * split <= 2048) split *= 2;
+    while (vec && 2 * split * nch <= CM_MW && chunks * 2 * split <= 2048) split *= 2;
     const int hpb = split > 1 ? 1 : CM_AW / nch;
     void* cargs[] = {&k, &dv, &nch, &split};
     const dim3 grid((p->heads + hpb - 1) / hpb, p->rows, 1), block(64 * (split > 1 ? nch * split : CM_AW), 1, 1);
 #define QMLA_CMB(H, NC) \
-    (split > 1 ? (const void*)&combine_bal_kernel<H, NC, true> : (const void*)&combine_bal_kernel<H, NC, false>)
-    const void* fn = k.part_h ? (nc == 4 ? QMLA_CMB(true, 4) : QMLA_CMB(true, 8))
-                              : (nc == 4 ? QMLA_CMB(false, 4) : QMLA_CMB(false, 8));
+    (split > 1 ? (const void*)&combine_bal_kernel<H, NC, true, true> : (const void*)&combine_bal_kernel<H, NC, false, true>)
+    const void* fn = !vec      ? (k.part_h ? (const void*)&combine_bal_kernel<true, 8, false, false>
+                                           : (const void*)&combine_bal_kernel<false, 8, false, false>)
+                     : k.part_h ? (nc == 4 ? QMLA_CMB(true, 4) : QMLA_CMB(true, 8))
+                                : (nc == 4 ? QMLA_CMB(false, 4) : QMLA_CMB(false, 8));
 #undef QMLA_CMB
     return launch(fn, grid, block, cargs, st);
   }
