@@ -825,25 +825,25 @@ __device__ __forceinline__ void merge_segments(const KParams& p, int64_t slot0, 
 }
 
 // H = fp16 partials without the fp8 scale, which is applied here; nch chunks of 64*NC columns per
-// row; `split` waves per chunk (1 unless SPLIT). Workgroups of nch*split waves (SPLIT: one head), or
-// of CM_AW waves that take the chunks of CM_AW / nch heads. VEC: rows of whole lane vectors, as every
+// row. SPLIT: 2^sh waves per chunk, workgroups of nch 2^sh waves and one head; else workgroups of CM_AW
+// waves, 2^sh >= nch of them for a head's chunks (no integer division by either: most rows of a large
+// batch were finished by one workgroup, and their waves only find that out). VEC: rows of whole lane vectors, as every
 // layout a decode kernel is compiled for; the combine entry point takes partials of any even width, which
 // are read by elements. Those loads in the same kernel took it from 43-94 VGPRs to 77-138, at 3 waves a
 // SIMD instead of 5 to 8, for rows that never use them: 700 rank-1792 bf16 requests of 150 tokens 33.0 us
 // with them and 28.0 without, 128 of 1500 17.3 / 15.2, 128 rank-1792 fp8 requests of 6000 17.5 / 14.2.
 template <bool H, int NC, bool SPLIT, bool VEC>
-__global__ __launch_bounds__(64 * (SPLIT ? CM_MW : CM_AW)) void combine_bal_kernel(const KParams p, int dv, int nch, int split) {
+__global__ __launch_bounds__(64 * (SPLIT ? CM_MW : CM_AW)) void combine_bal_kernel(const KParams p, int dv, int nch, int sh) {
   constexpr int CW = 64 * NC;
   const int row = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int req = row / p.qrows, jq = row - req * p.qrows;
+  const int req = p.qrows == 1 ? row : row / p.qrows, jq = row - req * p.qrows;
   // the wave's head, chunk of columns and, with SPLIT, share of the segments
-  const int hpb = SPLIT ? 1 : CM_AW / nch;
-  const int unit = SPLIT ? wv / split : wv, sub = SPLIT ? wv - unit * split : 0;
-  const int hh = SPLIT ? 0 : unit / nch, ch = SPLIT ? unit : unit - hh * nch;
-  const int head = (int)blockIdx.x * hpb + hh;
-  if (!SPLIT && (hh >= hpb || head >= p.heads)) return;
+  const int split = SPLIT ? 1 << sh : 1, low = wv & ((1 << sh) - 1), high = wv >> sh;
+  const int sub = SPLIT ? low : 0, ch = SPLIT ? high : low;
+  const int head = SPLIT ? (int)blockIdx.x : (int)blockIdx.x * (CM_AW >> sh) + high;
+  if (!SPLIT && (ch >= nch || head >= p.heads)) return;
   const float osc = H && p.k_scale ? *p.k_scale : 1.0f;
   const int chunk = p.plan[0];
   const int c0 = p.plan[2 + req], c1 = p.plan[3 + req];
@@ -1252,11 +1252,12 @@ static int run_combine(const qmla_decode_params* p, KParams& k, hipStream_t st) 
     // over 4; bf16 B 4, 96 chunks: 4.3 split over 8, 7.2 unsplit)
     const int nc = dv <= 256 && dv % 4 == 0 ? 4 : 8;
     const bool vec = dv % nc == 0;
-    int nch = (dv + 64 * nc - 1) / (64 * nc), split = 1;
+    int nch = (dv + 64 * nc - 1) / (64 * nc), split = 1, sh = 0;
     const int64_t chunks = (int64_t)p->rows * p->heads * nch;
     while (vec && 2 * split * nch <= CM_MW && chunks * 2 * split <= 2048) split *= 2;
-    const int hpb = split > 1 ? 1 : CM_AW / nch;
-    void* cargs[] = {&k, &dv, &nch, &split};
+    while ((1 << sh) < (split > 1 ? split : nch)) ++sh;   // nch <= 4: dv is at most 2048
+    const int hpb = split > 1 ? 1 : CM_AW >> sh;
+    void* cargs[] = {&k, &dv, &nch, &sh};
     const dim3 grid((p->heads + hpb - 1) / hpb, p->rows, 1), block(64 * (split > 1 ? nch * split : CM_AW), 1, 1);
 #define QMLA_CMB(H, NC) \
     (split > 1 ? (const void*)&combine_bal_kernel<H, NC, true, true> : (const void*)&combine_bal_kernel<H, NC, false, true>)
