@@ -754,16 +754,19 @@ __global__ __launch_bounds__(256) void combine_kernel(const KParams p, int dv) {
 // workgroups of 8 waves took 17 / 31 us for work that 4 waves each finish in 6) and the latency of its
 // dependent loads (plan, then partials). So a wave merges a chunk of 64*NC columns of one (row, head)
 // with 16 bytes a lane of fp16 partials (32 of fp32) and up to 8 segments in flight at once:
-//   SPLIT false  a wave merges its chunk alone, without LDS or a barrier (2 and 4 heads a wave, 4
-//                segments of each in flight: FP8 B 128 6.4 -> 8.4 us, GLA-g2 7.4 -> 10.0);
+//   SPLIT false  a wave merges its chunk alone, without LDS or a barrier (with 2 and 4 heads a wave and 4
+//                segments of each in flight FP8 B 128 took a third longer);
 //   SPLIT true   the segments of a chunk are dealt out over several waves, whose sums meet in LDS:
 //                for few rows, whose requests were split over many workgroups (one request of 1300
-//                tokens: 21 segments).
-// Combine launch before (256 threads for a row and 2 heads, 4 bytes a lane) and now: FP8 B 128 9.8 ->
-// 6.4 us, GLA-g2 11.2 -> 7.4, one request 8.6 -> 5.1, bf16 B 4 9.7 -> 4.3, 23 rank-768 requests 18.4 ->
-// 7.9, 19 rank-1792 requests 8.9 -> 8.4.
+//                tokens: 21 segments). Up to CM_ALONE segments, one batch of loads, a chunk's first
+//                wave merges them alone: 7 segments of one request, rank 512 / 256 4.0 -> 3.9 / 3.5 us,
+//                rank 1792 5.0 -> 4.4; 3 segments of 33 requests, rank 512 5.0 -> 4.2.
+// Combine launch before (256 threads for a row and 2 heads, 4 bytes a lane) and now, back to back in a
+// graph: FP8 B 128 8.7 -> 5.6 us, GLA-g2 10.4 -> 6.3, verify B 64 x 4 11.6 -> 7.4, one request 7.6 -> 4.3,
+// bf16 B 4 8.1 -> 4.4, 23 rank-768 requests 16.0 -> 6.1, 19 rank-1792 requests 7.4 -> 6.3.
 constexpr int CM_MW = 8;    // waves of a workgroup that splits chunks, at most
 constexpr int CM_AW = 4;    // waves of a workgroup that does not
+constexpr int CM_ALONE = 8; // segments of a chunk that one wave merges
 
 // merges segments s0, s0 + step, ... (NS of them; those past nseg weigh 0 and re-read the last one)
 // into the running (m, l, a) of columns col .. col + NC of partial row rl
@@ -866,14 +869,17 @@ __global__ __launch_bounds__(64 * (SPLIT ? CM_MW : CM_AW)) void combine_bal_kern
 #pragma unroll
   for (int c = 0; c < NC; ++c) a[c] = 0.f;
   const int lc = col < dv ? col : 0, rl = jq * p.heads + head;
-  merge_segments<H, NC, VEC>(p, (int64_t)w0 + req, rl, dv, lc, sub, split, nseg, m, l, a);
-  if constexpr (!SPLIT) {
+  // few segments: one wave merges its chunk alone (workgroup-uniform: the others leave here)
+  const bool alone = !SPLIT || nseg <= CM_ALONE;
+  if (SPLIT && alone && sub != 0) return;
+  merge_segments<H, NC, VEC>(p, (int64_t)w0 + req, rl, dv, lc, sub, alone ? 1 : split, nseg, m, l, a);
+  if (alone) {
     const float inv = inv_sum(osc, l);
 #pragma unroll
     for (int c = 0; c < NC; ++c)
       if (col + c < dv) store_out(p.out, p.out_dt, ob + col + c, a[c] * inv);
     if (ch == 0 && lane == 0 && p.lse) store_out(p.lse, p.lse_dt, lb, empty_sum(l) ? kNegInf : m + __logf(l));
-  } else {
+  } else if constexpr (SPLIT) {
     __shared__ float s_a[CM_MW][CW];
     __shared__ float s_m[CM_MW], s_l[CM_MW];
 #pragma unroll
@@ -1248,8 +1254,9 @@ static int run_combine(const qmla_decode_params* p, KParams& k, hipStream_t st) 
   if (p->num_splits == 0 && (dv & 1)) return QMLA_ERR_SHAPE;   // no row format has an odd number of columns
   if (p->num_splits == 0) {
     // columns a lane and chunks of columns per (row, head); a chunk is split over up to 8 waves while
-    // they stay within 2048, 8 a CU (23 rank-768 requests, 1104 chunks: 7.9 us unsplit, 10.8 split
-    // over 4; bf16 B 4, 96 chunks: 4.3 split over 8, 7.2 unsplit)
+    // they stay within 2048, 8 a CU of 256. bf16 B 4 (96 chunks): 4.4 us split over 8, 5.4 over 2; 23
+    // rank-768 requests (1104): 6.1 unsplit, 6.2 over 2, 7.6 over 4; bf16 B 64 (1536): 4.5 unsplit, 5.3
+    // over 2; 19 rank-1792 requests (1824): 6.3 and 8.1; FP8 B 128 (3072): 5.6 and 7.2
     const int nc = dv <= 256 && dv % 4 == 0 ? 4 : 8;
     const bool vec = dv % nc == 0;
     int nch = (dv + 64 * nc - 1) / (64 * nc), split = 1, sh = 0;
