@@ -590,7 +590,6 @@ __global__ __launch_bounds__(C::NTHR, 1) void ro_kernel(const KParams p) {
     else role_main<C, DMA>(p, sm, kscale, fixed, lo, hi, b0, c0, wr, len, bad);
     report_pages(p, bad);
   }
-  __builtin_amdgcn_wave_barrier();   // one exit for every path (no instruction)
 }
 
 typedef void (*RoFn)(const KParams);

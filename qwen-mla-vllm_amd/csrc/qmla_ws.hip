@@ -930,7 +930,6 @@ __global__ __launch_bounds__(C::NTHR, 1) void ws_kernel(const KParams p) {
     else role_main<C, VALUE>(p, sm, kscale, fixed, lo, hi, b0, c0, wr, hz, len, bad);
     report_pages(p, bad);
   }
-  __builtin_amdgcn_wave_barrier();   // one exit for every path (no instruction)
 }
 
 struct Inst {

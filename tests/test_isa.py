@@ -38,7 +38,7 @@ def _assembly(tmp_path, source):
 def _kernels(lines, pattern):
     starts = [i for i, l in enumerate(lines) if re.match(pattern, l)]
     for s in starts:
-        e = next(i for i in range(s, len(lines)) if "s_endpgm" in lines[i])
+        e = next(i for i in range(s, len(lines)) if lines[i].startswith(".Lfunc_end"))   # blocks may follow s_endpgm
         yield lines[s].split(":")[0], lines[s:e]
 
 
