@@ -758,9 +758,10 @@ __global__ __launch_bounds__(256) void combine_kernel(const KParams p, int dv) {
 //                segments of each in flight FP8 B 128 took a third longer);
 //   SPLIT true   the segments of a chunk are dealt out over several waves, whose sums meet in LDS:
 //                for few rows, whose requests were split over many workgroups (one request of 1300
-//                tokens: 21 segments). Up to CM_ALONE segments, one batch of loads, a chunk's first
-//                wave merges them alone: 7 segments of one request, rank 512 / 256 4.0 -> 3.9 / 3.5 us,
-//                rank 1792 5.0 -> 4.4; 3 segments of 33 requests, rank 512 5.0 -> 4.2.
+//                tokens: 21 segments). Rows of three or four chunks, where only two waves share one, merge
+//                up to CM_ALONE segments (one batch of loads) in the chunk's first wave: rank 1792, one
+//                request of 3 segments 4.7 -> 4.1 us, of 7 5.0 -> 4.4. In the narrower rows' kernel the
+//                second way costs 16 layers of one request of 21 segments 1.5 us of 261.
 // Combine launch before (256 threads for a row and 2 heads, 4 bytes a lane) and now, back to back in a
 // graph: FP8 B 128 8.7 -> 5.6 us, GLA-g2 10.4 -> 6.3, verify B 64 x 4 11.6 -> 7.4, one request 7.6 -> 4.3,
 // bf16 B 4 8.1 -> 4.4, 23 rank-768 requests 16.0 -> 6.1, 19 rank-1792 requests 7.4 -> 6.3.
@@ -835,7 +836,7 @@ __device__ __forceinline__ void merge_segments(const KParams& p, int64_t slot0, 
 // are read by elements. Those loads in the same kernel took it from 43-94 VGPRs to 77-138, at 3 waves a
 // SIMD instead of 5 to 8, for rows that never use them: 700 rank-1792 bf16 requests of 150 tokens 33.0 us
 // with them and 28.0 without, 128 of 1500 17.3 / 15.2, 128 rank-1792 fp8 requests of 6000 17.5 / 14.2.
-template <bool H, int NC, bool SPLIT, bool VEC>
+template <bool H, int NC, bool SPLIT, bool VEC, bool ALONE = false>
 __global__ __launch_bounds__(64 * (SPLIT ? CM_MW : CM_AW)) void combine_bal_kernel(const KParams p, int dv, int nch, int sh) {
   constexpr int CW = 64 * NC;
   const int row = blockIdx.y;
@@ -870,7 +871,7 @@ __global__ __launch_bounds__(64 * (SPLIT ? CM_MW : CM_AW)) void combine_bal_kern
   for (int c = 0; c < NC; ++c) a[c] = 0.f;
   const int lc = col < dv ? col : 0, rl = jq * p.heads + head;
   // few segments: one wave merges its chunk alone (workgroup-uniform: the others leave here)
-  const bool alone = !SPLIT || nseg <= CM_ALONE;
+  const bool alone = !SPLIT || (ALONE && nseg <= CM_ALONE);
   if (SPLIT && alone && sub != 0) return;
   merge_segments<H, NC, VEC>(p, (int64_t)w0 + req, rl, dv, lc, sub, alone ? 1 : split, nseg, m, l, a);
   if (alone) {
@@ -1266,10 +1267,13 @@ static int run_combine(const qmla_decode_params* p, KParams& k, hipStream_t st) 
     const int hpb = split > 1 ? 1 : CM_AW >> sh;
     void* cargs[] = {&k, &dv, &nch, &sh};
     const dim3 grid((p->heads + hpb - 1) / hpb, p->rows, 1), block(64 * (split > 1 ? nch * split : CM_AW), 1, 1);
+    const bool alone = nch > 2;   // see CM_ALONE
 #define QMLA_CMB(H, NC) \
     (split > 1 ? (const void*)&combine_bal_kernel<H, NC, true, true> : (const void*)&combine_bal_kernel<H, NC, false, true>)
     const void* fn = !vec      ? (k.part_h ? (const void*)&combine_bal_kernel<true, 8, false, false>
                                            : (const void*)&combine_bal_kernel<false, 8, false, false>)
+                     : split > 1 && alone ? (k.part_h ? (const void*)&combine_bal_kernel<true, 8, true, true, true>
+                                                      : (const void*)&combine_bal_kernel<false, 8, true, true, true>)
                      : k.part_h ? (nc == 4 ? QMLA_CMB(true, 4) : QMLA_CMB(true, 8))
                                 : (nc == 4 ? QMLA_CMB(false, 4) : QMLA_CMB(false, 8));
 #undef QMLA_CMB

@@ -25,6 +25,7 @@ LENS = [2500, 0, 130, 64, 65, 700]
     ("fp8", 768, 232, 24, 1, 1, 50, 64),     # ... unsplit
     ("bf16", 1792, 64, 24, 1, 1, 3, 60),     # 4 chunks: split 2
     ("bf16", 1792, 64, 24, 1, 1, 12, 60),    # ... unsplit
+    ("fp8", 1792, 232, 24, 1, 1, 6, 64),     # split 2, requests of 2 to 40 segments: one wave up to 8
     ("fp8", 512, 64, 24, 4, 2, 1, 256),      # 256 columns, 2 latent groups, verify rows: split 8
     ("fp8", 512, 64, 24, 4, 2, 24, 256),     # ... unsplit
 ])
