@@ -14,8 +14,10 @@ namespace qmla {
 
 constexpr int PLAN_TILE = 64;  // balancing granularity of the balanced plan (tokens)
 // plan tiles the balanced plan charges per request switch (see plan_tiles), per kernel family: the
-// warp-specialized and row-owner decode (measured: a piece's query load and output write cost about
-// two plan tiles of work), the per-group and column-split kernels (none)
+// warp-specialized and row-owner decode, for a piece's query load and output write, the per-group and
+// column-split kernels (none). At 1 / 2 / 3 tiles, whole call, alternating runs: GLA-g2 B 48 x 4 168.2 /
+// 167.2 / 168.7 us, verify B 64 x 4 358.8 / 356.8 / 356.5, bf16 B 64 221.2 / 220.6 / 222.6, the FP8 B 128
+// headline the same; 4 layers of 23 rank-768 requests 185.8 / 175.2 / 165.0
 constexpr int kPlanSwitchWs = 2, kPlanSwitchRo = 2, kPlanSwitchOther = 0;
 
 struct KParams {
@@ -351,9 +353,10 @@ __device__ __forceinline__ void store_out4(char* ptr, const f32x4& v) {
 // Stores one row's columns from 16x16 accumulator tiles of O^T = V^T . P^T: lane (lg, n) holds columns
 // 16cb + 4lg + i of row n, scaled by inv (num / the row's sum). e is the element offset of the row's
 // first column, live false for rows past the request's. A tile's columns go out in one 8- or 16-byte
-// store a lane and the output's type is branched on once. With O = P . V (a lane holding column n of
-// four rows) the same tiles took 64 stores of 2 or 4 bytes a lane in about 1000 basic blocks, 3.4 us
-// a piece; transposed in registers before the store, 2.3 us.
+// store a lane and the output's type is branched on once. A finished request of two row blocks, by
+// timestamps: 3.4 us with O = P . V (a lane holding column n of four rows: 64 stores of 2 or 4 bytes a lane
+// in about 1000 basic blocks), 2.3 us with that transposed in registers before the store, 2.0 us as it is
+// (0.35 for sums and addresses, 0.75 a row block).
 template <int CB>
 __device__ __forceinline__ void store_row(const RowOut& o, const f32x4 (&acc)[CB], float inv, int64_t e, bool live) {
   if (!live) return;
