@@ -58,8 +58,8 @@ def cache_write_params(kv_c: torch.Tensor, k_pe: torch.Tensor, kv_cache: torch.T
         raise ValueError("cache_write: fewer input rows than slots")
     if kv_c2.stride(-1) != 1 or k_pe2.stride(-1) != 1:
         raise ValueError("cache_write: rows must be contiguous in their last dimension")
-    if slots.dtype != torch.int64:
-        slots = slots.to(torch.int64)
+    if slots.dtype != torch.int64 or not slots.is_contiguous():
+        slots = slots.to(torch.int64).contiguous()
     p = _lib.CacheWriteParams()
     p.kv_c, p.kv_c_stride = kv_c2.data_ptr(), kv_c2.stride(0)
     p.k_pe, p.k_pe_stride = k_pe2.data_ptr(), k_pe2.stride(0)

@@ -140,6 +140,21 @@ def test_log8_code_of_every_bf16(gpu, copies):
     assert np.array_equal(got, np.tile(exp, (copies, 1)))
 
 
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_strided_slot_mapping(gpu, dtype):
+    """A slot mapping that is a column of a wider tensor: its own elements, not those beside them."""
+    import qmla
+    n = 90
+    kv_c, k_pe = _inputs(n, seed=5)
+    wide = torch.full((n, 3), -1, dtype=dtype)
+    wide[:, 1] = torch.randperm(8 * 16, generator=torch.Generator().manual_seed(5))[:n]
+    cache = torch.zeros(8, 16, 600, dtype=torch.bfloat16, device=gpu)
+    qmla.cache_write(kv_c.to(gpu), k_pe.to(gpu), cache, wide.to(gpu)[:, 1], rope_w=ROPE, rms_heads=H, kv_fp8=False,
+                     rms="bf16")
+    got = cache.cpu().view(-1, 600)[wide[:, 1].long()]
+    assert torch.equal(got, torch.cat([kv_c, k_pe], 1))
+
+
 def test_bf16_rows_copied(gpu):
     import qmla
     n, P, pages = 50, 16, 10
