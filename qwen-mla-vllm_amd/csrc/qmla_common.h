@@ -75,9 +75,7 @@ inline void page_magic(int d, uint32_t& mul, int& sh) {
   sh = 31 + l;
   mul = (uint32_t)((((uint64_t)1 << sh) + (uint64_t)d - 1) / (uint64_t)d);
 }
-__host__ __device__ __forceinline__ uint32_t magic_div(uint32_t x, uint32_t mul, int sh) {
-  return (uint32_t)(((uint64_t)x * mul) >> sh);
-}
+__host__ __device__ __forceinline__ uint64_t magic_div(uint32_t x, uint32_t mul, int sh) { return ((uint64_t)x * mul) >> sh; }
 __device__ __forceinline__ int page_div(const KParams& p, int x) { return (int)magic_div((uint32_t)x, p.page_mul, p.page_sh); }
 
 // A block-table entry checked against the page bound: an entry outside [0, page_bound) reads page 0
