@@ -831,11 +831,12 @@ __device__ __forceinline__ void merge_segments(const KParams& p, int64_t slot0, 
 // H = fp16 partials without the fp8 scale, which is applied here; nch chunks of 64*NC columns per
 // row. SPLIT: 2^sh waves per chunk, workgroups of nch 2^sh waves and one head; else workgroups of CM_AW
 // waves, 2^sh >= nch of them for a head's chunks (no integer division by either: most rows of a large
-// batch were finished by one workgroup, and their waves only find that out). VEC: rows of whole lane vectors, as every
-// layout a decode kernel is compiled for; the combine entry point takes partials of any even width, which
-// are read by elements. Those loads in the same kernel took it from 43-94 VGPRs to 77-138, at 3 waves a
-// SIMD instead of 5 to 8, for rows that never use them: 700 rank-1792 bf16 requests of 150 tokens 33.0 us
-// with them and 28.0 without, 128 of 1500 17.3 / 15.2, 128 rank-1792 fp8 requests of 6000 17.5 / 14.2.
+// batch were finished by one workgroup, and their waves only find that out). VEC: rows of whole lane
+// vectors, as every layout a decode kernel is compiled for; the combine entry point takes partials of any
+// even width, which are read by elements. Those loads in the same kernel took it from 43-94 VGPRs to
+// 77-138, at 3 waves a SIMD instead of 5 to 8, for rows that never use them: 700 rank-1792 bf16 requests of
+// 150 tokens 33.0 us with them and 28.0 without (21.9 without the divisions too), 128 of 1500 17.3 / 15.2,
+// 128 rank-1792 fp8 requests of 6000 17.5 / 14.2. ALONE: see CM_ALONE above.
 template <bool H, int NC, bool SPLIT, bool VEC, bool ALONE = false>
 __global__ __launch_bounds__(64 * (SPLIT ? CM_MW : CM_AW)) void combine_bal_kernel(const KParams p, int dv, int nch, int sh) {
   constexpr int CW = 64 * NC;

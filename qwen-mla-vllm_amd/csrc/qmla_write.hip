@@ -522,8 +522,8 @@ __device__ __forceinline__ uint4 dequant8(const uint2 raw, float sc) {
 // first conversion. The same values as gather_kernel.
 //
 // What bounds it: as write_rows_kernel, the waves and their chain (sequence, page, row) below some 20000
-// rows, memory above. 20000 rows of rank 512 / 768 / 1792: 13.4 / 14.3 / 21.6 us at one row a wave
-// (gather_kernel), 11.0 / 13.5 / 20.7 at two rows, 10.6 / 14.7 / 23.6 at four; 65536 rows 34.8 / 35.9 /
+// rows, memory above. 16384 rows of rank 512 / 768 / 1792: 11.4 / 12.6 / 18.7 us at one row a wave
+// (gather_kernel), 9.3 / 12.3 / 18.1 at two rows, 9.3 / 13.1 / 20.6 at four; 65536 rows 34.8 / 35.9 /
 // 59.6 at one, 26.5 / 35.1 / 62.2 at two, 24.2 / 34.9 / 65.7 at four.
 template <int DT, int R, int NF>
 __global__ __launch_bounds__(256) void gather_rows_kernel(const GParams p) {
